@@ -517,7 +517,7 @@ int32_t qwh_decoder_forward_rows(qwh_decoder *decoder, const uint32_t *tokens, c
  * logits stay on the device). An empty prompt, or audio pads that do not
  * match audio_steps, give QWH_E_SHAPE_MISMATCH (the reference's
  * UnexpectedShape / PromptMismatch). The positions are processed together,
- * in chunks of 256: each layer's products run over all of them, their cache
+ * in chunks of up to 512: each layer's products run over all of them, their cache
  * rows are appended, then each attends to the cache rows up to its own.
  * Layer matrices without a matrix-core form run their per-token GEMV once
  * over a chunk's rows (f32 / f16, q5 / q8, and q4 rows its fused GEMV

@@ -452,6 +452,21 @@ int32_t qwh_linear(qwh_ctx *ctx, uint64_t matrix, const float *x_dev, uint32_t c
     QWH_TRY(check_device_ptr(ctx, out_dev, "out"));
     if (((uintptr_t)x_dev & 15u) != 0) return fail(ctx, QWH_E_INVALID_ARGUMENT, "x must be 16-byte aligned");
     if (m->rows == 0) return QWH_OK;
+    // Many tokens: 32-token tiles on the f16 matrix cores (the q5 shapes that
+    // the forms below refuse stay refused).
+    if (gemm_rows_preferred(*m, tokens) &&
+        (m->format != QWH_FORMAT_Q5 || gemv_batch_supported(*m) || gemv_b8_supported(m->format, m->rows, m->cols))) {
+        QWH_TRY(ensure_workspace(ctx, ctx->digits, rows_activation_bytes(tokens, cols)));
+        const size_t parts = rows_partial_bytes(ctx->cus, tokens, *m);
+        if (parts) QWH_TRY(ensure_workspace(ctx, ctx->scratch, parts));
+        RowsInput in;
+        in.x = x_dev;
+        QWH_TRY(check_hip(ctx, launch_prep_rows(ctx->stream, in, m->format, tokens, cols, ctx->digits.ptr), "prep rows"));
+        RowsOutput out;
+        out.out = out_dev;
+        if (parts) out.partials = static_cast<float *>(ctx->scratch.ptr);
+        return check_hip(ctx, launch_gemm_rows(ctx->stream, ctx->cus, ctx->digits.ptr, *m, tokens, out), "gemm rows");
+    }
     if (m->format == QWH_FORMAT_Q4) {
         if (tokens >= 2) {
             // Several tokens: int8 digit planes, then one matrix-core pass

@@ -233,6 +233,39 @@ hipError_t launch_gemv_batch_parts(hipStream_t s, const void *digits, const Matr
                                    float *partials, const BatchNorm &norm = BatchNorm{},
                                    uint32_t *slices_used = nullptr);
 
+// Quantized matrices times many rows of f32 activations (gemm_rows.hip): the
+// activations split once into two f16 terms per value (rows_activation_bytes),
+// in the order that `format`'s decode takes, then 32-token tiles on the f16
+// matrix cores. K a multiple of 64, at least 256.
+constexpr uint32_t kRowsMaxSlices = 8;
+struct RowsInput {
+    // F32: x. RmsNorm: x * weight / rms(x) (x first plus `sums`, also stored
+    // to sums.x_out). Pairs: siluMul of the gate / up rows in `sums`.
+    enum Form { F32, RmsNorm, Pairs } form = F32;
+    const float *x = nullptr, *weight = nullptr;
+    float eps = 0.0f;
+    PartialSums sums;
+};
+struct RowsOutput {
+    float *out = nullptr;
+    const float *residual = nullptr;    // out = residual + W x (may be out)
+    bool pairs = false;                 // out = siluMul of row pairs
+    float *partials = nullptr;          // rows_partial_bytes, needed for a K split
+};
+bool gemm_rows_supported(const Matrix &w);
+// The form is the faster one for this many tokens.
+bool gemm_rows_preferred(const Matrix &w, uint32_t tokens);
+size_t rows_activation_bytes(uint32_t tokens, uint32_t cols);
+size_t rows_partial_bytes(int cus, uint32_t tokens, const Matrix &w);
+// Rows of at most 8192 values; F32 rows of any length.
+hipError_t launch_prep_rows(hipStream_t s, const RowsInput &in, int format, uint32_t tokens, uint32_t cols, void *acts);
+// out = W x. A K split leaves its partial sums [slice][token][row] in
+// out.partials: added by a second launch (plain products only), or, with
+// `slices_left`, by the caller, who finds their number there (0: the output
+// is complete).
+hipError_t launch_gemm_rows(hipStream_t s, int cus, const void *acts, const Matrix &w, uint32_t tokens,
+                            const RowsOutput &out, uint32_t *slices_left = nullptr);
+
 // q4 / q5 GEMM with bf16 activations (gemm.hip). `scratch` holds the split-K
 // partials: gemm_scratch_bytes (0 when the tiles alone fill the device).
 size_t gemm_scratch_bytes(int cus, uint32_t tokens, const Matrix &w);

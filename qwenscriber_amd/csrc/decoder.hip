@@ -450,13 +450,14 @@ struct qwh_decoder {
     float *parts = nullptr;
     bool split_parts = false;
     uint32_t slices_o = 0, slices_gu = 0, slices_down = 0, slices_qkv = 0;
-    // qwh_decoder_prefill's buffers, for up to kPrefillChunk prompt positions
+    // qwh_decoder_prefill's buffers, for the prompt positions of one chunk
     // of one sequence, allocated at its first call.
     struct PrefillBuffers {
         float *hidden = nullptr, *qkv = nullptr, *attn = nullptr, *rope = nullptr, *parts = nullptr;
         float *wide = nullptr;  // the rows form's siluMul(gate, up) rows
         void *digits = nullptr, *attn_scratch = nullptr, *arg_scratch = nullptr;
         size_t attn_scratch_bytes = 0;
+        uint32_t rows = 0;               // positions the buffers hold
         uint32_t *staged_dev = nullptr;  // tokens, audio row indices, positions
         uint32_t *id_dev = nullptr;
         uint32_t *host = nullptr;        // pinned: the same three arrays, then the id
@@ -1405,7 +1406,8 @@ int32_t qwh_decoder_forward_rows(qwh_decoder *d, const uint32_t *tokens, const f
 
 namespace {
 
-constexpr uint32_t kPrefillChunk = 256;
+constexpr uint32_t kPrefillChunk = 512;     // at most (the staging's stride)
+constexpr uint32_t kPrefillTileChunk = 256;  // of the forms other than prefill_chunk_gemm
 
 // How a prompt runs through the layers:
 //   MatrixCores  every layer product has a matrix-core form, o / gate|up /
@@ -1418,6 +1420,23 @@ constexpr uint32_t kPrefillChunk = 256;
 // The first two also need the attention and the prefill append for the head
 // shape.
 enum class PrefillForm { MatrixCores, Rows, Positions };
+
+// The rows from which a MatrixCores chunk runs on the 32-token tiles of the
+// f16 matrix cores (prefill_chunk_gemm) rather than the 16-token ones, by the
+// layers' shapes; ~0u: never. The two meet near 6e9 multiply-adds a layer: a
+// 1.7B decoder's prompt (50.3M weights a layer) took 2.96 ms with 16-token
+// tiles and 3.06 with these at 128 positions, 3.85 and 3.72 at 192; a 0.6B
+// one's (15.7M) 2.91 and 3.03 at 256, 5.27 and 4.12 at 402.
+uint32_t gemm_rows_from(const qwh_decoder *d) {
+    const qwh_decoder::Layer &L = d->layers[0];
+    uint64_t weights = 0;
+    for (const Matrix *m : {&L.qkv, &L.o, &L.gu, &L.down}) {
+        if (m->cols < 256 || m->cols > 8192) return ~0u;
+        weights += (uint64_t)m->rows * m->cols;
+    }
+    const uint64_t rows = (6000000000ull + weights - 1) / weights;
+    return rows > kPrefillChunk ? ~0u : (uint32_t)rows;
+}
 
 bool rows_gemv_supported(const Matrix &m) {
     if (is_dense_format(m.format)) return gemv_dense_supported(m.format, m.cols);
@@ -1444,7 +1463,11 @@ int32_t prefill_buffers(qwh_decoder *d) {
     qwh_decoder::PrefillBuffers &pf = d->pf;
     if (pf.host) return QWH_OK;
     const qwh_decoder_config &c = d->c;
-    const size_t P = kPrefillChunk;
+    // (Shapes alone: a matrix bound in another format later still fits.)
+    const uint32_t from = gemm_rows_from(d);
+    pf.rows = from == ~0u ? kPrefillTileChunk : kPrefillChunk;
+    const size_t P = pf.rows;
+    const uint32_t tiled = std::min((uint32_t)P, from);  // rows of a chunk on 16-token tiles, at most
     const uint32_t qkv_n = d->qw + 2 * d->kvw;
     const uint32_t widest = std::max(std::max(c.hidden, c.ffn), d->qw);
     QWH_TRY(dalloc(d, sizeof(float) * P * c.hidden, reinterpret_cast<void **>(&pf.hidden)));
@@ -1452,21 +1475,25 @@ int32_t prefill_buffers(qwh_decoder *d) {
     QWH_TRY(dalloc(d, sizeof(float) * P * d->qw, reinterpret_cast<void **>(&pf.attn)));
     QWH_TRY(dalloc(d, sizeof(float) * P * c.ffn, reinterpret_cast<void **>(&pf.wide)));
     QWH_TRY(dalloc(d, sizeof(float) * P * c.head_dim, reinterpret_cast<void **>(&pf.rope)));
-    QWH_TRY(dalloc(d, batch_digit_bytes((uint32_t)P, widest), &pf.digits));
+    QWH_TRY(dalloc(d, std::max(batch_digit_bytes(tiled, widest), rows_activation_bytes((uint32_t)P, widest)),
+                   &pf.digits));
     const qwh_decoder::Layer &L0 = d->layers[0];
     size_t parts = 4;
-    for (const Matrix *m : {&L0.qkv, &L0.o, &L0.gu, &L0.down})
-        parts = std::max(parts, batch_partial_bytes((uint32_t)P, *m));
+    for (const Matrix *m : {&L0.qkv, &L0.o, &L0.gu, &L0.down}) {
+        parts = std::max(parts, batch_partial_bytes(tiled, *m));
+        // (The 32-token tiles' K split depends on the chunk's rows.)
+        for (uint32_t n = from; n <= P; ++n) parts = std::max(parts, rows_partial_bytes(d->ctx->cus, n, *m));
+    }
     QWH_TRY(dalloc(d, parts, reinterpret_cast<void **>(&pf.parts)));
     // The attention records: sized per chunk (the range count depends on
     // the chunk's rows and positions), grown by prefill_chunk when a chunk
     // needs more.
     pf.attn_scratch_bytes = 0;
     QWH_TRY(dalloc(d, argmax_scratch_bytes(1, c.vocab), &pf.arg_scratch));
-    QWH_TRY(dalloc(d, 3 * 4 * P, reinterpret_cast<void **>(&pf.staged_dev)));
+    QWH_TRY(dalloc(d, 3 * 4 * (size_t)kPrefillChunk, reinterpret_cast<void **>(&pf.staged_dev)));
     QWH_TRY(dalloc(d, 4, reinterpret_cast<void **>(&pf.id_dev)));
     void *host = nullptr;
-    QWH_TRY(check_hip(d->ctx, hipHostMalloc(&host, 4 * (3 * P + 8), hipHostMallocDefault), "pinned prefill staging"));
+    QWH_TRY(check_hip(d->ctx, hipHostMalloc(&host, 4 * (3 * (size_t)kPrefillChunk + 8), hipHostMallocDefault), "pinned prefill staging"));
     pf.host = static_cast<uint32_t *>(host);
     return QWH_OK;
 }
@@ -1664,6 +1691,74 @@ int32_t prefill_chunk(qwh_decoder *d, uint32_t seq, uint32_t first, uint32_t n, 
     return check_hip(d->ctx, launch_prep_batch(s, fin, n, H, pf.digits, &pending), "prefill final");
 }
 
+// prefill_chunk for enough rows to fill 32-token tiles: each product's input
+// is split into f16 terms by one pass (which also adds the previous product's
+// K slices to the residual stream, or forms siluMul of gate and up), o and
+// down add the residual themselves where K is not split.
+int32_t prefill_chunk_gemm(qwh_decoder *d, uint32_t seq, uint32_t first, uint32_t n, const float *audio_rows, bool last) {
+    qwh_decoder::PrefillBuffers &pf = d->pf;
+    const qwh_decoder_config &c = d->c;
+    hipStream_t s = d->ctx->stream;
+    const uint32_t H = c.hidden;
+    const uint32_t *tokens_dev = pf.staged_dev, *index_dev = pf.staged_dev + kPrefillChunk;
+    embed_prompt_kernel<<<n, 256, 0, s>>>(tokens_dev, index_dev, d->embed.format,
+                                          reinterpret_cast<const uint16_t *>(d->embed.scales), d->embed.data, H,
+                                          pf.hidden, first, d->rope_cos, d->rope_sin, c.head_dim / 2, pf.rope,
+                                          audio_rows);
+    QWH_TRY(check_hip(d->ctx, hipGetLastError(), "prefill embedding"));
+    PartialSums pending{};  // the last product's slices, not yet in pf.hidden
+    auto split = [&](const RowsInput &in, const Matrix &w) {
+        return check_hip(d->ctx, launch_prep_rows(s, in, w.format, n, w.cols, pf.digits), "prefill prep");
+    };
+    auto normed = [&](const float *norm) {
+        RowsInput in;
+        in.form = RowsInput::RmsNorm;
+        in.x = pf.hidden;
+        in.weight = norm;
+        in.eps = c.eps;
+        in.sums = pending;
+        return in;
+    };
+    // W * the split rows into `out`, or, with K split, into pf.parts, whose
+    // slice count is returned in `slices`.
+    auto product = [&](const Matrix &w, float *out, const float *residual, bool pairs, uint32_t &slices,
+                       const char *what) {
+        RowsOutput o;
+        o.out = out;
+        o.residual = residual;
+        o.pairs = pairs;
+        o.partials = pf.parts;
+        return check_hip(d->ctx, launch_gemm_rows(s, d->ctx->cus, pf.digits, w, n, o, &slices), what);
+    };
+    for (uint32_t l = 0; l < c.layers; ++l) {
+        qwh_decoder::Layer &L = d->layers[l];
+        uint32_t slices = 0;
+        QWH_TRY(split(normed(L.attn_norm), L.qkv));
+        QWH_TRY(product(L.qkv, pf.qkv, nullptr, false, slices, "prefill q|k|v"));
+        QWH_TRY(prefill_attention(d, seq, first, n, l, slices ? pf.parts : pf.qkv, slices ? slices : 1, nullptr));
+        RowsInput in;
+        in.x = pf.attn;
+        QWH_TRY(split(in, L.o));
+        QWH_TRY(product(L.o, pf.hidden, pf.hidden, false, slices, "prefill o"));
+        pending = slices ? PartialSums{pf.parts, slices, H, false, pf.hidden} : PartialSums{};
+        QWH_TRY(split(normed(L.ffn_norm), L.gu));
+        QWH_TRY(product(L.gu, pf.wide, nullptr, true, slices, "prefill gate|up"));
+        RowsInput wide;
+        wide.x = pf.wide;
+        if (slices) {
+            wide.form = RowsInput::Pairs;
+            wide.sums = PartialSums{pf.parts, slices, 2 * c.ffn, true, nullptr};
+        }
+        QWH_TRY(split(wide, L.down));
+        QWH_TRY(product(L.down, pf.hidden, pf.hidden, false, slices, "prefill down"));
+        pending = slices ? PartialSums{pf.parts, slices, H, false, pf.hidden} : PartialSums{};
+    }
+    if (!last || !pending.slices) return QWH_OK;
+    // The residual stream after the last layer (its split is not used).
+    return check_hip(d->ctx, launch_prep_rows(s, normed(d->final_norm), QWH_FORMAT_Q4, n, H, pf.digits),
+                     "prefill final");
+}
+
 }  // namespace
 
 int32_t qwh_decoder_prefill(qwh_decoder *d, uint32_t seq, const uint32_t *tokens, uint32_t count,
@@ -1722,8 +1817,10 @@ int32_t qwh_decoder_prefill(qwh_decoder *d, uint32_t seq, const uint32_t *tokens
     qwh_decoder::PrefillBuffers &pf = d->pf;
     hipStream_t s = d->ctx->stream;
     uint32_t audio_index = 0;
-    for (uint32_t c0 = 0; c0 < count; c0 += kPrefillChunk) {
-        const uint32_t n = std::min(kPrefillChunk, count - c0);
+    const uint32_t chunk = form == PrefillForm::MatrixCores ? pf.rows : kPrefillTileChunk;
+    const uint32_t gemm_from = gemm_rows_from(d);
+    for (uint32_t c0 = 0; c0 < count; c0 += chunk) {
+        const uint32_t n = std::min(chunk, count - c0);
         // The pinned staging is reused per chunk: the previous chunk's copy
         // has completed (the stream was synchronized below).
         uint32_t *h_tokens = pf.host, *h_index = pf.host + kPrefillChunk, *h_pos = pf.host + 2 * kPrefillChunk;
@@ -1736,7 +1833,10 @@ int32_t qwh_decoder_prefill(qwh_decoder *d, uint32_t seq, const uint32_t *tokens
         QWH_TRY(check_hip(d->ctx, hipMemcpyAsync(pf.staged_dev, pf.host, 3 * 4 * (size_t)kPrefillChunk,
                                                  hipMemcpyHostToDevice, s), "prefill tokens"));
         const bool last = c0 + n == count;
-        if (form == PrefillForm::MatrixCores) QWH_TRY(prefill_chunk(d, seq, pos0 + c0, n, audio_rows_dev, last));
+        if (form == PrefillForm::MatrixCores && n >= gemm_from)
+            QWH_TRY(prefill_chunk_gemm(d, seq, pos0 + c0, n, audio_rows_dev, last));
+        else if (form == PrefillForm::MatrixCores)
+            QWH_TRY(prefill_chunk(d, seq, pos0 + c0, n, audio_rows_dev, last));
         else QWH_TRY(prefill_chunk_rows(d, seq, pos0 + c0, n, audio_rows_dev));
         if (last) {
             // decoder.zig:332 argmaxLogits of the last position.
