@@ -452,6 +452,12 @@ int32_t qwh_linear(qwh_ctx *ctx, uint64_t matrix, const float *x_dev, uint32_t c
     QWH_TRY(check_device_ptr(ctx, out_dev, "out"));
     if (((uintptr_t)x_dev & 15u) != 0) return fail(ctx, QWH_E_INVALID_ARGUMENT, "x must be 16-byte aligned");
     if (m->rows == 0) return QWH_OK;
+    if (gemv_tokens_preferred(*m, tokens)) {
+        GemvInput in;
+        in.mode = GemvInput::F32;
+        in.x = x_dev;
+        return check_hip(ctx, launch_gemv_tokens(ctx->stream, ctx->cus, in, *m, tokens, out_dev), "gemv tokens");
+    }
     // Many tokens: 32-token tiles on the f16 matrix cores (the q5 shapes that
     // the forms below refuse stay refused).
     if (gemm_rows_preferred(*m, tokens) &&

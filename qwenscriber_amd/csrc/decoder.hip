@@ -440,6 +440,7 @@ struct qwh_decoder {
     bool planned = false;
     bool fused = true;  // every q4 GEMV forms its own activations (no norm / prep kernels)
     bool batched = false;  // batch > 1: int8 digit planes + matrix-core GEMV
+    bool head_batched = false;  // the same for the lm_head
     // Per-token q4 GEMVs (fused, not batched): the embedding gathered by the
     // first q | k | v GEMV, the argmax partials formed by the lm_head GEMV.
     bool fold_embed = false, fold_argmax = false;
@@ -568,12 +569,22 @@ int32_t plan_step(qwh_decoder *d) {
         batch_form = batch_form && gemv_batch_supported(*m);
     }
     d->fused = q4_fused;
+    // A few sequences of a small model: the layers on the per-token GEMVs
+    // (with every q4 one forming its own activations), the long lm_head still
+    // on the matrix cores.
+    const qwh_decoder::Layer &first = d->layers[0];
+    uint64_t weights = 0;
+    for (const Matrix *m : {&first.qkv, &first.o, &first.gu, &first.down}) weights += (uint64_t)m->rows * m->cols;
+    d->head_batched = batch_form;
+    if (batch_form && q4_fused && gemv_tokens_preferred_layer(first.gu.format, weights, d->batch)) {
+        batch_form = false;
+        d->head_batched = !gemv_tokens_preferred(d->lm_head, d->batch);
+    }
     d->batched = batch_form;
     const bool per_token_q4 = q4_fused && !batch_form;
-    const qwh_decoder::Layer &first = d->layers[0];
     d->fold_embed = per_token_q4 && first.qkv.format == QWH_FORMAT_Q4 &&
                     gemv_q4_source_supported(GemvInput::Embed, first.qkv.rows, first.qkv.cols);
-    d->fold_argmax = per_token_q4 && d->lm_head.format == QWH_FORMAT_Q4;
+    d->fold_argmax = per_token_q4 && !d->head_batched && d->lm_head.format == QWH_FORMAT_Q4;
     d->split_parts = false;
     d->slices_o = d->slices_gu = d->slices_down = d->slices_qkv = 0;
     if (d->batched) {
@@ -608,14 +619,14 @@ int32_t enqueue_step(qwh_decoder *d, bool want_logits) {
     // residual stream's pending update, or the gate / up pairs).
     PartialSums pending;
     auto gemv = [&](GemvInput::Mode mode, const float *x, const float *norm, const Matrix &w, float *out,
-                    const float *residual, bool pairs) -> hipError_t {
+                    const float *residual, bool pairs, bool batched) -> hipError_t {
         GemvInput in;
         in.mode = mode;
         in.x = x;
         in.norm = norm;
         in.eps = c.eps;
         in.pairs = pairs;
-        if (d->batched) {
+        if (batched) {
             if (mode != GemvInput::Digits) {  // Digits: the planes are already in batch_digits
                 const hipError_t e = launch_prep_batch(s, in, B, w.cols, d->batch_digits, &pending);
                 pending = PartialSums{};
@@ -683,7 +694,7 @@ int32_t enqueue_step(qwh_decoder *d, bool want_logits) {
             in.rope_now = d->rope_now;
             err = launch_gemv_q4_src(s, ctx->cus, in, L.qkv, B, d->qkv, nullptr);
         } else {
-            err = gemv(GemvInput::RmsNorm, d->hidden, L.attn_norm, L.qkv, d->qkv, nullptr, false);
+            err = gemv(GemvInput::RmsNorm, d->hidden, L.attn_norm, L.qkv, d->qkv, nullptr, false, d->batched);
         }
         if (err != hipSuccess) break;
         // Per-head norms, RoPE, the cache append and the attention itself
@@ -751,12 +762,12 @@ int32_t enqueue_step(qwh_decoder *d, bool want_logits) {
             continue;
         }
         err = gemv(d->batched ? GemvInput::Digits : GemvInput::F32, d->attn, nullptr, L.o, d->hidden, d->hidden,
-                   false);
+                   false, d->batched);
         if (err != hipSuccess) break;
         // gate | up rows interleaved: the GEMV writes siluMul(gate, up).
-        err = gemv(GemvInput::RmsNorm, d->hidden, L.ffn_norm, L.gu, d->gu, nullptr, true);
+        err = gemv(GemvInput::RmsNorm, d->hidden, L.ffn_norm, L.gu, d->gu, nullptr, true, d->batched);
         if (err != hipSuccess) break;
-        err = gemv(GemvInput::F32, d->gu, nullptr, L.down, d->hidden, d->hidden, false);
+        err = gemv(GemvInput::F32, d->gu, nullptr, L.down, d->hidden, d->hidden, false, d->batched);
     }
     if (err == hipSuccess) {
         if (want_logits) {
@@ -775,7 +786,8 @@ int32_t enqueue_step(qwh_decoder *d, bool want_logits) {
                           ? launch_gemv_q4_src(s, ctx->cus, in, d->lm_head, B, d->logits, nullptr)
                           : hipErrorInvalidValue;
             } else {
-                err = gemv(GemvInput::RmsNorm, d->hidden, d->final_norm, d->lm_head, d->logits, nullptr, false);
+                err = gemv(GemvInput::RmsNorm, d->hidden, d->final_norm, d->lm_head, d->logits, nullptr, false,
+                           d->head_batched);
                 if (err == hipSuccess)
                     argmax_partial_kernel<<<dim3(d->arg_parts, B), 256, 0, s>>>(d->logits, c.vocab, d->arg_per_block,
                                                                                  d->arg_v, d->arg_i);
@@ -1481,8 +1493,8 @@ int32_t prefill_buffers(qwh_decoder *d) {
     size_t parts = 4;
     for (const Matrix *m : {&L0.qkv, &L0.o, &L0.gu, &L0.down}) {
         parts = std::max(parts, batch_partial_bytes(tiled, *m));
-        // (The 32-token tiles' K split depends on the chunk's rows.)
-        for (uint32_t n = from; n <= P; ++n) parts = std::max(parts, rows_partial_bytes(d->ctx->cus, n, *m));
+        // (The 32-token tiles' K split depends on their number.)
+        for (uint32_t n = P; n >= from; n -= 32) parts = std::max(parts, rows_partial_bytes(d->ctx->cus, n, *m));
     }
     QWH_TRY(dalloc(d, parts, reinterpret_cast<void **>(&pf.parts)));
     // The attention records: sized per chunk (the range count depends on

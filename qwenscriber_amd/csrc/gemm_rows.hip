@@ -592,7 +592,7 @@ RowsPlan rows_plan(int cus, uint32_t tokens, uint32_t rows, uint32_t cols, uint3
             const uint32_t per_cu = (uint32_t)((units * ((tiles + tt - 1) / tt) + die_cus - 1) / die_cus);
             float us = (float)std::min(p.slice_groups, groups) * step_us(tt, per_cu);
             if (p.slices > 1)
-                us += (folded ? 0.5f : 3.0f) + (float)p.slices * (float)tokens * (float)rows * 8.0f / 4.5e6f;
+                us += (folded ? 0.5f : 3.0f) + (float)p.slices * (float)(tiles * kTile) * (float)rows * 8.0f / 4.5e6f;
             if (least == 0.0f || us < least) least = us, best = p;
         }
     return best;
