@@ -6,6 +6,7 @@
 #include <cstdio>
 #include <cstring>
 
+#include <algorithm>
 #include <initializer_list>
 #include <mutex>
 #include <vector>
@@ -1100,13 +1101,12 @@ int32_t qwh_conv3x3s2_gelu(qwh_ctx *ctx, float *out_dev, const float *in_dev, co
     QWH_TRY(check_device_ptr(ctx, weights_dev, "weights"));
     QWH_TRY(check_device_ptr(ctx, bias_dev, "bias"));
     if (conv_mfma_supported(in_channels, in_height, in_width)) {
-        // The matrix-core form: the weights prepared into the context's
-        // scratch, then the convolution.
-        QWH_TRY(ensure_workspace(ctx, ctx->scratch, conv_mfma_prep_bytes(out_channels, in_channels)));
-        QWH_TRY(check_hip(ctx, launch_conv_mfma_prep(ctx->stream, weights_dev, out_channels, in_channels,
-                                                     ctx->scratch.ptr), "conv weight prep"));
-        return check_hip(ctx, launch_conv3x3s2_gelu_mfma(ctx->stream, out_dev, in_dev, ctx->scratch.ptr, bias_dev, batch,
-                                                         out_channels, in_channels, in_height, in_width),
+        // The matrix-core form, its weights and activation terms prepared in
+        // the context's scratch.
+        QWH_TRY(ensure_workspace(ctx, ctx->scratch, conv_mfma_bytes(batch, out_channels, in_channels, in_height, in_width)));
+        return check_hip(ctx, launch_conv3x3s2_gelu_mfma(ctx->stream, ctx->cus, out_dev, in_dev, weights_dev, bias_dev, batch,
+                                                         out_channels, in_channels, in_height, in_width,
+                                                         ctx->scratch.ptr),
                          "conv3x3 stride 2");
     }
     return check_hip(ctx, launch_conv3x3s2_gelu(ctx->stream, out_dev, in_dev, weights_dev, bias_dev, batch, out_channels,
@@ -1161,24 +1161,27 @@ int32_t qwh_audio_frontend(qwh_ctx *ctx, const qwh_audio_frontend_weights *w, co
     const size_t p3 = (size_t)downsample * bins * chunk_steps;
     const uint32_t group = chunks < 32 ? chunks : 32;
     auto align = [](size_t n) { return (n + 63) & ~(size_t)63; };  // floats: 256-byte aligned pieces
-    const size_t off1 = align(group * mel_plane), off2 = off1 + align(group * p1), off3 = off2 + align(group * p2);
+    // conv2 and conv3 on the matrix cores where their shapes allow, with
+    // the intermediate planes in that form's layout; else f32 planes, each
+    // stage in the form it has.
+    ConvTower tower;
+    tower.weights[0] = w->conv1_weight, tower.weights[1] = w->conv2_weight, tower.weights[2] = w->conv3_weight;
+    tower.bias[0] = w->conv1_bias, tower.bias[1] = w->conv2_bias, tower.bias[2] = w->conv3_bias;
+    tower.bins = mel_bins, tower.chunk_frames = chunk_frames, tower.channels = downsample, tower.group = group;
+    const bool fused = conv_tower_supported(tower);
+    const size_t off1 = fused ? 0 : align(group * mel_plane), off2 = off1 + (fused ? 0 : align(group * p1));
+    const size_t off3 = off2 + (fused ? 0 : align(group * p2));
     const size_t off_flat = off3 + align(group * p3);
-    // conv2 / conv3 on the matrix cores where their shapes allow: their
-    // weights prepared once per call after the planes.
+    const size_t off_tower = off_flat + align((size_t)group * chunk_steps * features);
     const bool mfma2 = conv_mfma_supported(downsample, h1, w1), mfma3 = conv_mfma_supported(downsample, h2, w2);
-    const size_t prep_floats = align(conv_mfma_prep_bytes(downsample, downsample) / sizeof(float));
-    const size_t off_prep2 = off_flat + align((size_t)group * chunk_steps * features);
-    const size_t off_prep3 = off_prep2 + (mfma2 ? prep_floats : 0);
-    const size_t total = off_prep3 + (mfma3 ? prep_floats : 0);
+    const size_t tower_bytes = fused ? conv_tower_bytes(tower)
+                                     : std::max(mfma2 ? conv_mfma_bytes(group, downsample, downsample, h1, w1) : 0,
+                                                mfma3 ? conv_mfma_bytes(group, downsample, downsample, h2, w2) : 0);
+    const size_t total = off_tower + align(tower_bytes / sizeof(float) + 1);
     QWH_TRY(ensure_workspace(ctx, ctx->front, total * sizeof(float)));
     float *ws = static_cast<float *>(ctx->front.ptr);
     hipStream_t s = ctx->stream;
-    if (mfma2)
-        QWH_TRY(check_hip(ctx, launch_conv_mfma_prep(s, w->conv2_weight, downsample, downsample, ws + off_prep2),
-                          "conv2 weight prep"));
-    if (mfma3)
-        QWH_TRY(check_hip(ctx, launch_conv_mfma_prep(s, w->conv3_weight, downsample, downsample, ws + off_prep3),
-                          "conv3 weight prep"));
+    if (fused) QWH_TRY(check_hip(ctx, launch_conv_tower_prep(s, tower, log_mel_dev, frames, ws + off_tower), "front-end prep"));
     if (!ctx->front_table.ptr || ctx->front_table_steps != chunk_steps || ctx->front_table_width != d_model) {
         // addSinusoidalPosition (model.zig:751-763) for the steps of a chunk,
         // in f64 on the host, narrowed to f32 as the reference does; built
@@ -1206,20 +1209,25 @@ int32_t qwh_audio_frontend(qwh_ctx *ctx, const qwh_audio_frontend_weights *w, co
         const uint32_t count = chunks - c0 < group ? chunks - c0 : group;
         const uint32_t row0 = c0 * chunk_steps;  // every chunk before the last is whole
         const uint32_t rows = (uint32_t)(steps - row0 < (uint64_t)count * chunk_steps ? steps - row0 : count * chunk_steps);
-        QWH_TRY(check_hip(ctx, launch_gather_chunks(s, log_mel_dev, mel_bins, frames, chunk_frames, c0, count, ws),
-                          "front-end chunks"));
-        QWH_TRY(check_hip(ctx, launch_conv3x3s2_gelu(s, ws + off1, ws, w->conv1_weight, w->conv1_bias, count, downsample,
-                                                     1, mel_bins, chunk_frames), "conv1"));
-        QWH_TRY(check_hip(ctx, mfma2 ? launch_conv3x3s2_gelu_mfma(s, ws + off2, ws + off1, ws + off_prep2,
-                                                                  w->conv2_bias, count, downsample, downsample, h1, w1)
-                                     : launch_conv3x3s2_gelu(s, ws + off2, ws + off1, w->conv2_weight, w->conv2_bias,
-                                                             count, downsample, downsample, h1, w1),
-                          "conv2"));
-        QWH_TRY(check_hip(ctx, mfma3 ? launch_conv3x3s2_gelu_mfma(s, ws + off3, ws + off2, ws + off_prep3,
-                                                                  w->conv3_bias, count, downsample, downsample, h2, w2)
-                                     : launch_conv3x3s2_gelu(s, ws + off3, ws + off2, w->conv3_weight, w->conv3_bias,
-                                                             count, downsample, downsample, h2, w2),
-                          "conv3"));
+        if (fused) {
+            QWH_TRY(check_hip(ctx, launch_conv_tower(s, ctx->cus, tower, log_mel_dev, frames, c0, count, ws + off3, ws + off_tower),
+                              "convolutions"));
+        } else {
+            auto conv = [&](float *to, const float *from, const uint16_t *weights, const float *bias, uint32_t cin,
+                            uint32_t h, uint32_t width, bool mfma) {
+                return mfma ? launch_conv3x3s2_gelu_mfma(s, ctx->cus, to, from, weights, bias, count, downsample, cin, h, width,
+                                                         ws + off_tower)
+                            : launch_conv3x3s2_gelu(s, to, from, weights, bias, count, downsample, cin, h, width);
+            };
+            QWH_TRY(check_hip(ctx, launch_gather_chunks(s, log_mel_dev, mel_bins, frames, chunk_frames, c0, count, ws),
+                              "front-end chunks"));
+            QWH_TRY(check_hip(ctx, conv(ws + off1, ws, w->conv1_weight, w->conv1_bias, 1, mel_bins, chunk_frames, false),
+                              "conv1"));
+            QWH_TRY(check_hip(ctx, conv(ws + off2, ws + off1, w->conv2_weight, w->conv2_bias, downsample, h1, w1, mfma2),
+                              "conv2"));
+            QWH_TRY(check_hip(ctx, conv(ws + off3, ws + off2, w->conv3_weight, w->conv3_bias, downsample, h2, w2, mfma3),
+                              "conv3"));
+        }
         QWH_TRY(check_hip(ctx, launch_pack_steps(s, ws + off3, downsample, bins, chunk_steps, rows, ws + off_flat),
                           "front-end flatten"));
         float *out = encoder_dev + (size_t)row0 * d_model;

@@ -349,13 +349,27 @@ hipError_t launch_kv_append_q8(hipStream_t s, const float *key, const float *val
 hipError_t launch_conv3x3s2_gelu(hipStream_t s, float *out, const float *in, const uint16_t *weights, const float *bias,
                                  uint32_t batch, uint32_t out_ch, uint32_t in_ch, uint32_t h, uint32_t w);
 // The matrix-core form for input channels a multiple of 16 (planes small
-// enough for its LDS patch: conv_mfma_supported): weights prepared once per
-// weight set into `wprep` (conv_mfma_prep_bytes) by launch_conv_mfma_prep.
+// enough for its LDS patch: conv_mfma_supported); scratch holds
+// conv_mfma_bytes.
 bool conv_mfma_supported(uint32_t in_ch, uint32_t h, uint32_t w);
-size_t conv_mfma_prep_bytes(uint32_t out_ch, uint32_t in_ch);
-hipError_t launch_conv_mfma_prep(hipStream_t s, const uint16_t *weights, uint32_t out_ch, uint32_t in_ch, void *wprep);
-hipError_t launch_conv3x3s2_gelu_mfma(hipStream_t s, float *out, const float *in, const void *wprep, const float *bias,
-                                     uint32_t batch, uint32_t out_ch, uint32_t in_ch, uint32_t h, uint32_t w);
+size_t conv_mfma_bytes(uint32_t batch, uint32_t out_ch, uint32_t in_ch, uint32_t h, uint32_t w);
+hipError_t launch_conv3x3s2_gelu_mfma(hipStream_t s, int cus, float *out, const float *in, const uint16_t *weights,
+                                      const float *bias, uint32_t batch, uint32_t out_ch, uint32_t in_ch, uint32_t h,
+                                      uint32_t w, void *scratch);
+// The tower's three convolutions over chunks of chunk_frames frames of a
+// log-mel, up to `group` chunks at a time, where conv2 and conv3 have that
+// form: the intermediate planes stay in its layout. launch_conv_tower_prep
+// once per call, then each run of chunks to out [count][channels][h3][w3].
+struct ConvTower {
+    const uint16_t *weights[3] = {};
+    const float *bias[3] = {};
+    uint32_t bins = 0, chunk_frames = 0, channels = 0, group = 0;
+};
+bool conv_tower_supported(const ConvTower &c);
+size_t conv_tower_bytes(const ConvTower &c);
+hipError_t launch_conv_tower_prep(hipStream_t s, const ConvTower &c, const float *mel, uint32_t frames, void *scratch);
+hipError_t launch_conv_tower(hipStream_t s, int cus, const ConvTower &c, const float *mel, uint32_t frames, uint32_t first,
+                             uint32_t count, float *out, void *scratch);
 hipError_t launch_gather_chunks(hipStream_t s, const float *mel, uint32_t bins, uint32_t frames, uint32_t chunk_frames,
                                 uint32_t first, uint32_t count, float *out);
 hipError_t launch_pack_steps(hipStream_t s, const float *conv3, uint32_t channels, uint32_t bins, uint32_t steps_per_chunk,

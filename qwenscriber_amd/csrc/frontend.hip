@@ -18,7 +18,7 @@
 // 4 positions in f32 FMAs (the reference sums each input channel's nine taps
 // before adding them to the output; the order here differs, within f32
 // rounding), then adds the bias and applies GELU (the reference's erf fit).
-#include <type_traits>
+#include <algorithm>
 
 #include "common.h"
 #include "device.h"
@@ -105,208 +105,442 @@ __global__ __launch_bounds__(256) void conv3x3s2_gelu_kernel(const ConvArgs a) {
 
 // ---- Matrix-core form (input channels a multiple of 16) ----
 //
-// The convolution as an implicit GEMM on v_mfma_f32_32x32x16_bf16: rows are
+// The convolution as an implicit GEMM on v_mfma_f32_32x32x16_f16: rows are
 // output channels, columns are output positions (row-major over the output
 // plane), and the reduction runs over (tap, input channel) in stages of 16
-// input channels, one 16-deep MFMA step per tap. Both operands are split into
-// two bf16 terms: a weight (f16, 11 significant bits) is exactly hi + lo
-// (hi = its bf16 rounding, lo = the exact remainder, at most 4 bits); an
-// activation is hi + lo with hi its bf16 rounding and lo the bf16 rounding of
-// the exact remainder (|x - hi - lo| <= 2^-17 |x|). The four products are
-// accumulated in f32 by the MFMA, so each term is an exact product summed in
-// f32: within 2^-17 of the f32 convolution per term, no overflow range of its
-// own (bf16 has f32's exponent range).
+// input channels, one 16-deep MFMA step per tap. A weight is f16 as it is. An
+// activation is two f16 terms of x * s: hi its f16 rounding, lo the exact
+// remainder rounded to f16, with s a power of two for the whole tensor from a
+// bound on its largest magnitude, |x * s| < 2^15. So a value keeps 22
+// significant bits, and nothing above 2^-40 of the bound is lost; the
+// products are exact and summed in f32 by the matrix core. (Two bf16 terms of
+// both operands, without a scale, took four products a tap and kept 2^-17.)
 //
-// Workgroup: 128 output channels (four wavefronts of 32) x 64 positions (two
-// 32-column MFMA tiles per wavefront, so each weight operand serves both).
-// Per stage the 64 positions' input rows (at most 2 * ceil(63 / ow) + 3 of
-// them, zero padding included) x 16 channels go into LDS as
-// [row][col][channel] in both terms, double buffered, the next stage's values
-// loaded into registers while this one multiplies. Weights come prepared
-// [stage][tap][term][oc][16] (conv_mfma_prep_kernel) and each wavefront loads
-// its 32 rows' 18 operands one stage ahead. (32-position workgroups measured
-// 1.33 ms for the 30 s front end against 1.15 ms: every position tile reads
-// the weights again.)
-typedef __bf16 cbf16x8 __attribute__((ext_vector_type(8)));
-typedef __bf16 cbf16x2 __attribute__((ext_vector_type(2)));
+// The terms are stored once by whoever makes the activations (the "halves"
+// layout): [image][stage][plane][row][parity][slot] 16-byte words of 8
+// channels, plane = 2 * term + channel half, rows and columns padded by one
+// zero on each side and the padded columns split by parity. A tap of stride 2
+// reads one parity, so the 32 positions of an operand are consecutive words:
+// the patch is copied to LDS as it is, and read without bank conflicts or
+// tests for the border.
+//
+// Workgroup: 256 output channels (four wavefronts of 64) x 64 positions (or 32,
+// where the grid is small: launch_mfma); a wavefront's 64 x 64 tile takes eight products from four LDS words and two
+// weight words a lane. A stage's patch (at most 2 * ceil(63 / ow) + 3 rows) is
+// copied by global-to-LDS loads one stage ahead, and a tap's weights, stored
+// in operand order, are loaded a whole stage before their use. Bound by the
+// matrix cores (about 40 % of their rate, the LDS reads at half of theirs) and
+// by the last, partly empty wave of workgroups; 30 s of audio, 480 channels:
+// conv2 (64 x 50 planes) 706 -> 253 us, conv3 204 -> 82 us.
+typedef _Float16 ch8 __attribute__((ext_vector_type(8)));
+typedef _Float16 ch4 __attribute__((ext_vector_type(4)));
 typedef float cf32x16 __attribute__((ext_vector_type(16)));
+typedef uint32_t cu4 __attribute__((ext_vector_type(4)));
 
-constexpr int kMfOc = 128;       // output channels per workgroup
-constexpr int kMfPos = 64;       // output positions per workgroup (two 32-column MFMA tiles)
-constexpr int kMfNt = kMfPos / 32;
+constexpr int kMfOc = 256;       // output channels per workgroup, 64 per wavefront
+constexpr int kMfPos = 64;       // output positions per workgroup at most (one or two 32-column MFMA tiles)
 constexpr int kMfIc = 16;        // input channels per stage
-constexpr int kMfIcPad = 16;     // channel stride of a patch cell (bf16)
-constexpr int kMfRounds = 4;     // patch items per thread at most (256 threads)
-constexpr size_t kMfLdsMax = 80 * 1024;  // the patch buffers' LDS, two workgroups per CU
+constexpr int kMfRounds = 9;     // patch words per thread at most
 
-struct ConvMfmaArgs {
-    float *out;                  // [batch][out_ch][oh * ow]
-    const float *in;             // [batch][in_ch][h][w]
-    const uint16_t *wprep;       // [in_ch / 16][9][2][oc_pad][16] bf16 bits
-    const float *bias;
-    uint32_t out_ch, oc_pad, in_ch, h, w, oh, ow, positions;
-    uint32_t patch_rows, patch_cols;
+// A tensor in the halves layout: padded planes of (h + 2) rows x 2 parities x
+// slots words.
+struct HalvesPlane {
+    uint32_t slots, words;       // of a row and parity; of a plane
 };
 
-// Prepared weights: f16 -> f32 (exact), hi = bf16(w), lo = bf16(w - hi)
-// (exact), laid out for the A operand; rows past out_ch are zero.
-__global__ void conv_mfma_prep_kernel(const uint16_t *weights, uint32_t out_ch, uint32_t oc_pad, uint32_t in_ch,
-                                      uint16_t *wprep) {
-    const uint64_t n = (uint64_t)oc_pad * in_ch * 9;
-    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x) {
-        const uint32_t icl = (uint32_t)(i % kMfIc);
-        const uint32_t oc = (uint32_t)((i / kMfIc) % oc_pad);
-        const uint32_t tap = (uint32_t)((i / ((uint64_t)kMfIc * oc_pad)) % 9);
-        const uint32_t stage = (uint32_t)(i / ((uint64_t)kMfIc * oc_pad * 9));
-        const uint32_t ic = stage * kMfIc + icl;
-        const float v = oc < out_ch ? dev::f16_bits_to_f32(weights[((size_t)oc * in_ch + ic) * 9 + tap]) : 0.0f;
-        const __bf16 hi = (__bf16)v;
-        const __bf16 lo = (__bf16)(v - (float)hi);
-        const size_t base = (((size_t)stage * 9 + tap) * 2) * oc_pad;
-        wprep[(base + oc) * kMfIc + icl] = __builtin_bit_cast(uint16_t, hi);
-        wprep[(base + oc_pad + oc) * kMfIc + icl] = __builtin_bit_cast(uint16_t, lo);
+__host__ __device__ inline HalvesPlane halves_plane(uint32_t h, uint32_t w) {
+    const uint32_t slots = (w + 3) / 2;
+    return {slots, (h + 2) * 2 * slots};
+}
+
+struct ConvMfmaArgs {
+    const uint8_t *in;           // halves
+    const uint8_t *wprep;        // [stage][tap][oc / 32][lane][8] f16
+    const float *bias;
+    const float *scales;         // input: 2^-e; halves output: also its 2^e
+    float *out;                  // [batch][out_ch][oh * ow] f32, or null
+    uint8_t *halves;             // the output in the halves layout, or null
+    uint32_t out_ch, oc_tiles, stages, h, w, oh, ow, positions;
+    uint32_t patch_rows, pos_tiles, units, oc_blocks;
+};
+
+// The two terms of v * s.
+__device__ __forceinline__ void split_half(float v, float s, _Float16 &hi, _Float16 &lo) {
+    const float x = v * s;
+    hi = (_Float16)x;
+    const float rest = x - (float)hi;
+    lo = fabsf(rest) < __builtin_inff() ? (_Float16)rest : (_Float16)0.0f;  // (inf and NaN are hi's)
+}
+
+// s_waitcnt operand: at most N vector memory operations and no LDS operation
+// outstanding.
+template <int N>
+constexpr int kConvWait = (N & 15) | (7 << 4) | ((N >> 4) << 14);
+// The same for vector memory alone.
+template <int N>
+constexpr int kConvLoads = kConvWait<N> | (15 << 8);
+
+// NT: 32-position tiles; R: rounds of 256 patch words.
+template <int NT, int R, bool HALVES>
+__global__ __launch_bounds__(256, 2) void conv3x3s2_gelu_mfma_kernel(const ConvMfmaArgs a) {
+    __shared__ cu4 patch[2][R * 256];
+    const int t = threadIdx.x;
+    const int lane = t & 63, wave = t >> 6;
+    const int half = lane >> 5;
+    // Consecutive workgroups run on the eight dies in turn: a position tile's
+    // channel blocks stay on one die, next to each other.
+    const uint32_t die = blockIdx.x & 7, at = blockIdx.x >> 3;
+    const uint32_t unit = at / a.oc_blocks * 8 + die;
+    if (unit >= a.units) return;
+    const uint32_t b = unit / a.pos_tiles, p0 = unit % a.pos_tiles * (32 * NT);
+    const uint32_t oc0 = (at % a.oc_blocks) * kMfOc + wave * 64;
+    const HalvesPlane in_plane = halves_plane(a.h, a.w);
+    const uint32_t slots = in_plane.slots;
+    const uint32_t patch_plane = a.patch_rows * 2 * slots;  // words of a patch plane
+    const uint32_t r_first = p0 / a.ow;
+
+    if (HALVES && p0 == 0) {
+        // The output planes' zero border (this workgroup's channels, once per
+        // image): the first and last row, and in the others what is left and
+        // right of the columns.
+        const HalvesPlane o = halves_plane(a.oh, a.ow);
+        const uint32_t first = (at % a.oc_blocks) * (kMfOc / kMfIc);
+        const uint32_t count = min((uint32_t)(kMfOc / kMfIc), a.out_ch / kMfIc - first) * 4;
+        cu4 *to = reinterpret_cast<cu4 *>(a.halves) + ((size_t)b * (a.out_ch / kMfIc) + first) * 4 * o.words;
+        for (uint32_t i = t; i < o.words; i += 256) {
+            const uint32_t row = i / (2 * o.slots), rest = i % (2 * o.slots);
+            const uint32_t col = 2 * (rest % o.slots) + rest / o.slots;
+            if (row >= 1 && row <= a.oh && col >= 1 && col <= a.ow) continue;
+            for (uint32_t p = 0; p < count; ++p) to[(size_t)p * o.words + i] = cu4{0, 0, 0, 0};
+        }
+    }
+
+    // Patch words t, t + 256, ...: their source within a stage (the last word
+    // again past the patch, the last row again past the plane: both unused).
+    uint32_t from[R];
+#pragma unroll
+    for (int k = 0; k < R; ++k) {
+        const uint32_t u = min((uint32_t)(t + 256 * k), 4 * patch_plane - 1);
+        const uint32_t plane = u / patch_plane, rem = u % patch_plane;
+        const uint32_t row = min(2 * r_first + rem / (2 * slots), a.h + 1);
+        from[k] = plane * in_plane.words + row * 2 * slots + rem % (2 * slots);
+    }
+    const cu4 *image = reinterpret_cast<const cu4 *>(a.in) + (size_t)b * a.stages * 4 * in_plane.words;
+    auto copy_patch = [&](uint32_t stage, int buf) __attribute__((always_inline)) {
+        const cu4 *src = image + (size_t)stage * 4 * in_plane.words;
+#pragma unroll
+        for (int k = 0; k < R; ++k)
+            __builtin_amdgcn_global_load_lds(
+                reinterpret_cast<const __attribute__((address_space(1))) uint32_t *>(
+                    reinterpret_cast<uintptr_t>(src + from[k])),
+                reinterpret_cast<__attribute__((address_space(3))) uint32_t *>(
+                    reinterpret_cast<uintptr_t>(&patch[buf][wave * 64 + 256 * k])), 16, 0, 0);
+    };
+    // B operand: this lane's position (column lane % 32) and channel half.
+    uint32_t cell[NT];
+#pragma unroll
+    for (int j = 0; j < NT; ++j) {
+        const uint32_t p = min(p0 + 32 * j + (lane & 31), a.positions - 1);  // (past the plane: never stored)
+        cell[j] = half * patch_plane + 2 * (p / a.ow - r_first) * 2 * slots + p % a.ow;
+    }
+    // A operand: weights of oc0 + 32 i + lane % 32, channels 8 half .. + 7.
+    // (A wavefront past the channels multiplies the last ones' and stores
+    // nothing: a branch around its products would make the compiler wait for
+    // every load in flight at each stage.)
+    const cu4 *weights = reinterpret_cast<const cu4 *>(a.wprep) + (size_t)min(oc0 / 32, a.oc_tiles - 2) * 64 + lane;
+    const size_t tap_words = (size_t)a.oc_tiles * 64;
+    ch8 wa[9][2];
+    auto load_tap = [&](uint32_t stage, int tap) __attribute__((always_inline)) {
+        const cu4 *src = weights + ((size_t)stage * 9 + tap) * tap_words;
+        wa[tap][0] = __builtin_bit_cast(ch8, src[0]);
+        wa[tap][1] = __builtin_bit_cast(ch8, src[64]);
+        __builtin_amdgcn_sched_barrier(0);  // (else it sinks to the stage's end)
+    };
+    cf32x16 acc[2][NT] = {};
+    copy_patch(0, 0);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int tap = 0; tap < 9; ++tap) load_tap(0, tap);
+    for (uint32_t s = 0; s < a.stages; ++s) {
+        const int buf = s & 1;
+        const uint32_t next = min(s + 1, a.stages - 1);
+        // This stage's patch has landed (the 18 weight words a lane loaded
+        // after it may still travel), in every wavefront after the barrier;
+        // the other buffer was last read before it.
+        __builtin_amdgcn_s_waitcnt(kConvWait<18>);
+        __builtin_amdgcn_s_barrier();
+        copy_patch(next, buf ^ 1);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int tap = 0; tap < 9; ++tap) {
+            // This tap's weights: the 16 words of the other taps and R of the
+            // patch were loaded since, and loads complete in order. (Left to
+            // itself the compiler waits for everything once a copy to LDS is
+            // in flight.)
+            __builtin_amdgcn_s_waitcnt(kConvLoads<16 + R>);
+            const uint32_t step = (2 * (tap / 3) + (tap % 3 & 1)) * slots + (tap % 3 >> 1);
+#pragma unroll
+            for (int term = 0; term < 2; ++term) {
+                ch8 x[NT];
+#pragma unroll
+                for (int j = 0; j < NT; ++j)
+                    x[j] = __builtin_bit_cast(ch8, patch[buf][cell[j] + term * 2 * patch_plane + step]);
+#pragma unroll
+                for (int i = 0; i < 2; ++i)
+#pragma unroll
+                    for (int j = 0; j < NT; ++j)
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(wa[tap][i], x[j], acc[i][j], 0, 0, 0);
+            }
+            load_tap(next, tap);
+        }
+    }
+    __builtin_amdgcn_s_waitcnt(kConvWait<0>);  // (the last copy, unused, before the LDS is given back)
+    if (oc0 >= a.out_ch) return;
+    // Value r of a lane: output channel 8 (r / 4) + 4 half + r % 4 of the
+    // tile's 32, position column lane % 32.
+    const float inverse = a.scales[1];
+    const float up = HALVES ? a.scales[2] : 0.0f;
+    const HalvesPlane o = halves_plane(a.oh, a.ow);
+#pragma unroll
+    for (int j = 0; j < NT; ++j) {
+        const uint32_t pos = p0 + 32 * j + (lane & 31);
+        if (pos >= a.positions) continue;
+        const uint32_t row = pos / a.ow + 1, col = pos % a.ow + 1;
+        const uint32_t word = (row * 2 + (col & 1)) * o.slots + (col >> 1);
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const uint32_t oc = oc0 + 32 * i + 8 * q + 4 * half;
+                if (oc >= a.out_ch) continue;
+                float y[4];
+#pragma unroll
+                for (int k = 0; k < 4; ++k)
+                    y[k] = dev::gelu(a.bias[min(oc + k, a.out_ch - 1)] + acc[i][j][4 * q + k] * inverse);
+                if constexpr (HALVES) {
+                    ch4 hi, lo;
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) {
+                        _Float16 p, l;
+                        split_half(y[k], up, p, l);
+                        hi[k] = p, lo[k] = l;
+                    }
+                    // (Channels oc .. oc + 3 are half of a word of eight.)
+                    uint8_t *to = a.halves + ((((size_t)b * (a.out_ch / kMfIc) + oc / kMfIc) * 4 + (q & 1)) * o.words +
+                                              word) * 16 + 8 * half;
+                    *reinterpret_cast<ch4 *>(to) = hi;
+                    *reinterpret_cast<ch4 *>(to + (size_t)2 * o.words * 16) = lo;
+                } else {
+#pragma unroll
+                    for (int k = 0; k < 4; ++k)
+                        if (oc + k < a.out_ch) a.out[((size_t)b * a.out_ch + oc + k) * a.positions + pos] = y[k];
+                }
+            }
     }
 }
 
-__global__ __launch_bounds__(256) void conv3x3s2_gelu_mfma_kernel(const ConvMfmaArgs a) {
-    extern __shared__ __attribute__((aligned(16))) uint16_t patch_lds[];
-    const int t = threadIdx.x;
-    const int lane = t & 63;
-    const int wave = t >> 6;
-    const uint32_t oc0 = blockIdx.x * kMfOc + wave * 32;
-    const uint32_t p0 = blockIdx.y * kMfPos;
-    const uint32_t b = blockIdx.z;
-    const uint32_t cells = a.patch_rows * a.patch_cols;
-    const uint32_t term_elems = cells * kMfIcPad;          // one term of one buffer
-    const uint32_t r_first = p0 / a.ow;
-    const int in_r0 = 2 * (int)r_first - 1;                // input row of patch row 0
-    const float *in = a.in + (size_t)b * a.in_ch * a.h * a.w;
-    const uint32_t stages = a.in_ch / kMfIc;
+// What a call prepares: each convolution's weights in operand order with the
+// sum of magnitudes per output channel (a workgroup per channel; channels
+// past out_ch are zero), and the partial maxima of |x| over finite values of
+// an input (the workgroups after them).
+struct ConvWeightsJob {
+    const uint16_t *weights;     // [out_ch][in_ch][9] f16 bits
+    uint8_t *wprep;
+    float *norms;                // [oc_pad]
+    uint32_t out_ch, oc_pad, in_ch;
+};
 
-    // B operand: this lane's position (column lane % 32) and channel half.
-    uint32_t cell0[kMfNt];
+struct ConvPrepArgs {
+    ConvWeightsJob job[2];
+    const float *x;
+    uint64_t count;
+    float *partial;
+    uint32_t partials;
+};
+
+constexpr int kPrepIc = 512;
+
+__global__ __launch_bounds__(256) void conv_prep_kernel(const ConvPrepArgs a) {
+    __shared__ uint16_t rows[kPrepIc * 9];
+    __shared__ float red[4];
+    uint32_t block = blockIdx.x;
+    float v = 0.0f;
+    float *to;
+    const bool maxima = block >= a.job[0].oc_pad + a.job[1].oc_pad;
+    if (maxima) {
+        block -= a.job[0].oc_pad + a.job[1].oc_pad;
+        for (uint64_t i = (uint64_t)block * 256 + threadIdx.x; i < a.count; i += (uint64_t)a.partials * 256) {
+            const float m = fabsf(a.x[i]);
+            v = m < __builtin_inff() ? fmaxf(v, m) : v;
+        }
+        v = dev::wave_max(v);
+        to = a.partial + block;
+    } else {
+        const uint32_t n = block >= a.job[0].oc_pad ? 1 : 0;
+        const ConvWeightsJob &j = a.job[n];
+        const uint32_t oc = block - (n ? a.job[0].oc_pad : 0);
+        const uint16_t *row = j.weights + (size_t)min(oc, j.out_ch - 1) * j.in_ch * 9;
+        // A channel's weights through LDS, kPrepIc input channels at a time;
+        // items (stage, channel half, tap) are eight channels' of a tap.
+        for (uint32_t ic = 0; ic < j.in_ch; ic += kPrepIc) {
+            const uint32_t n = min((uint32_t)kPrepIc, j.in_ch - ic) * 9;
+            __syncthreads();
+            for (uint32_t i = threadIdx.x; i < n; i += 256) rows[i] = row[ic * 9 + i];
+            __syncthreads();
+            for (uint32_t i = threadIdx.x; i < n / 8; i += 256) {
+                const uint32_t tap = i % 9, h = i / 9 % 2, stage = ic / kMfIc + i / 18;
+                ch8 w;
 #pragma unroll
-    for (int j = 0; j < kMfNt; ++j) {
-        uint32_t p = p0 + 32 * j + (lane & 31);
-        if (p >= a.positions) p = a.positions - 1;              // (never stored)
-        const uint32_t oh = p / a.ow, ow = p % a.ow;
-        cell0[j] = (2 * (oh - r_first)) * a.patch_cols + 2 * ow;   // + kh * cols + kw
+                for (int k = 0; k < 8; ++k) {
+                    const uint16_t bits = rows[((i / 18) * kMfIc + 8 * h + k) * 9 + tap];
+                    w[k] = oc < j.out_ch ? __builtin_bit_cast(_Float16, bits) : (_Float16)0.0f;
+                    v += fabsf((float)w[k]);
+                }
+                *reinterpret_cast<ch8 *>(j.wprep + ((((size_t)stage * 9 + tap) * (j.oc_pad / 32) + oc / 32) * 64 +
+                                                    h * 32 + oc % 32) * 16) = w;
+            }
+        }
+        v = dev::wave_sum(v);
+        to = j.norms + oc;
     }
-    const uint32_t kq = (lane >> 5) * 8;
-    // A operand: output channel oc0 + lane % 32, channels kq .. kq + 7.
-    const uint16_t *wl = a.wprep + (size_t)(oc0 + (lane & 31)) * kMfIc + kq;
-    const size_t wtap = (size_t)2 * a.oc_pad * kMfIc;      // elements per tap (both terms)
-    const size_t wterm = (size_t)a.oc_pad * kMfIc;
-
-    // Patch items: (channel half, row, col); a thread takes items
-    // t, t + 256, ... (kMfRounds at most; the host checks 2 * cells fits).
-    float stage_v[kMfRounds][8];
-    auto load_patch = [&](uint32_t stage) {
-#pragma unroll
-        for (int k = 0; k < kMfRounds; ++k) {
-            const uint32_t item = t + 256 * k;
-            const uint32_t half = item / cells, cell = item % cells;
-            const int r = in_r0 + (int)(cell / a.patch_cols);
-            const int c = (int)(cell % a.patch_cols) - 1;
-            const bool inside = half < 2 && r >= 0 && r < (int)a.h && c >= 0 && c < (int)a.w;
-            const int rr = r < 0 ? 0 : (r >= (int)a.h ? (int)a.h - 1 : r);
-            const int cc = c < 0 ? 0 : (c >= (int)a.w ? (int)a.w - 1 : c);
-            const uint32_t ic = stage * kMfIc + (half < 2 ? half : 0) * 8;
-            const float *src = in + ((size_t)ic * a.h + rr) * a.w + cc;
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const float v = src[(size_t)j * a.h * a.w];   // (unconditional: clamped inside the plane)
-                stage_v[k][j] = inside ? v : 0.0f;
-            }
-        }
-    };
-    auto store_patch = [&](int buf) {
-        uint16_t *hi_base = patch_lds + (size_t)buf * 2 * term_elems;
-        uint16_t *lo_base = hi_base + term_elems;
-#pragma unroll
-        for (int k = 0; k < kMfRounds; ++k) {
-            const uint32_t item = t + 256 * k;
-            if (item >= 2 * cells) break;
-            const uint32_t half = item / cells, cell = item % cells;
-            uint32_t hw[4], lw[4];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const float x0 = stage_v[k][2 * j], x1 = stage_v[k][2 * j + 1];
-                const cbf16x2 h2 = {(__bf16)x0, (__bf16)x1};
-                const cbf16x2 l2 = {(__bf16)(x0 - (float)h2[0]), (__bf16)(x1 - (float)h2[1])};
-                hw[j] = __builtin_bit_cast(uint32_t, h2);
-                lw[j] = __builtin_bit_cast(uint32_t, l2);
-            }
-            const size_t at = (size_t)cell * kMfIcPad + half * 8;
-            *reinterpret_cast<uint4 *>(hi_base + at) = make_uint4(hw[0], hw[1], hw[2], hw[3]);
-            *reinterpret_cast<uint4 *>(lo_base + at) = make_uint4(lw[0], lw[1], lw[2], lw[3]);
-        }
-    };
-    cbf16x8 wa[2][9][2];  // [stage buffer][tap][term]
-    auto load_weights = [&](uint32_t stage, int buf) {
-        const uint16_t *src = wl + (size_t)stage * 9 * wtap;
-#pragma unroll
-        for (int tap = 0; tap < 9; ++tap)
-#pragma unroll
-            for (int term = 0; term < 2; ++term)
-                wa[buf][tap][term] = *reinterpret_cast<const cbf16x8 *>(src + tap * wtap + term * wterm);
-    };
-
-    cf32x16 acc[kMfNt] = {}, acc2[kMfNt] = {};
-    // One stage: the next stage's values and weights are loaded (the last
-    // stage reloads its own: the loads stay unconditional), this stage is
-    // multiplied out of LDS buffer BUF, and the next stage's values go into
-    // the other buffer; every wavefront read that buffer in the previous
-    // stage, before the barrier that ended it.
-    auto stage_step = [&](uint32_t s, auto buf_tag) {
-        constexpr int BUF = decltype(buf_tag)::value;
-        const uint32_t nxt = s + 1 < stages ? s + 1 : s;
-        load_patch(nxt);
-        load_weights(nxt, BUF ^ 1);
-        __builtin_amdgcn_sched_barrier(0);
-        const uint16_t *hb = patch_lds + (size_t)BUF * 2 * term_elems;
-        const uint16_t *lb = hb + term_elems;
-#pragma unroll
-        for (int tap = 0; tap < 9; ++tap) {
-#pragma unroll
-            for (int j = 0; j < kMfNt; ++j) {
-                const uint32_t cell = cell0[j] + (tap / 3) * a.patch_cols + (tap % 3);
-                const cbf16x8 bh = *reinterpret_cast<const cbf16x8 *>(hb + (size_t)cell * kMfIcPad + kq);
-                const cbf16x8 bl = *reinterpret_cast<const cbf16x8 *>(lb + (size_t)cell * kMfIcPad + kq);
-                // (Two accumulators, so consecutive products do not wait on
-                // each other's results.)
-                acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wa[BUF][tap][0], bh, acc[j], 0, 0, 0);
-                acc2[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wa[BUF][tap][0], bl, acc2[j], 0, 0, 0);
-                acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wa[BUF][tap][1], bh, acc[j], 0, 0, 0);
-                acc2[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wa[BUF][tap][1], bl, acc2[j], 0, 0, 0);
-            }
-        }
-        store_patch(BUF ^ 1);
-        __syncthreads();
-    };
-    load_patch(0);
-    load_weights(0, 0);
-    store_patch(0);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
     __syncthreads();
-    uint32_t s = 0;
-    for (; s + 1 < stages; s += 2) {
-        stage_step(s, std::integral_constant<int, 0>{});
-        stage_step(s + 1, std::integral_constant<int, 1>{});
-    }
-    if (s < stages) stage_step(s, std::integral_constant<int, 0>{});
-    // Value r of a lane: output channel row 8 (r / 4) + 4 (lane / 32) + r % 4
-    // of the wavefront's 32, position column lane % 32.
-#pragma unroll
-    for (int j = 0; j < kMfNt; ++j) {
-        const uint32_t pos = p0 + 32 * j + (lane & 31);
-        if (pos >= a.positions) continue;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const uint32_t oc = oc0 + 8 * (r / 4) + 4 * (lane >> 5) + (r % 4);
-            if (oc < a.out_ch)
-                a.out[((size_t)b * a.out_ch + oc) * a.positions + pos] =
-                    dev::gelu(a.bias[oc] + (acc[j][r] + acc2[j][r]));
+    if (threadIdx.x == 0)
+        *to = maxima ? fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3])) : (red[0] + red[1]) + (red[2] + red[3]);
+}
+
+// The tensors' scales {2^e, 2^-e} from bounds on their magnitudes: the first
+// from the partial maxima of the input -- that input itself, or (conv1) the
+// result of a one-channel convolution of it -- and the next from the first's
+// bound through a convolution's weight sums: |gelu(y)| <= |y| <= |bias| + sum
+// |w| * bound. (A bound a thousand times the largest value still keeps it to
+// 2^-30.)
+struct ConvScaleArgs {
+    const float *partial;
+    uint32_t partials;
+    const uint16_t *conv1;       // [channels][9] f16 bits, or null
+    const float *bias1, *norms2, *bias2;  // norms2 null: the first scale only
+    uint32_t channels;
+    float *scales;               // {s, 1 / s} of the first, then of the next
+};
+
+__device__ __forceinline__ float block_max_256(float v, float *red) {
+    v = dev::wave_max(v);
+    __syncthreads();
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+    __syncthreads();
+    return fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+}
+
+__global__ __launch_bounds__(256) void conv_scale_kernel(const ConvScaleArgs a) {
+    __shared__ float red[4];
+    float v = 0.0f;
+    for (uint32_t i = threadIdx.x; i < a.partials; i += 256) v = fmaxf(v, a.partial[i]);
+    float bound = block_max_256(v, red);
+    auto emit = [&](float m, float *to) {
+        // 2^e > m, with room for the bound's own rounding.
+        const int e = dev::chunk_exponent(fminf(m * 1.01f, 3.4e38f));
+        if (threadIdx.x == 0) to[0] = __builtin_ldexpf(1.0f, 15 - e), to[1] = __builtin_ldexpf(1.0f, e - 15);
+    };
+    if (a.conv1) {
+        v = 0.0f;
+        for (uint32_t c = threadIdx.x; c < a.channels; c += 256) {
+            float sum = 0.0f;
+            for (int k = 0; k < 9; ++k) sum += fabsf(dev::f16_bits_to_f32(a.conv1[(size_t)c * 9 + k]));
+            v = fmaxf(v, fabsf(a.bias1[c]) + sum * bound);
         }
+        bound = block_max_256(v, red);
+    }
+    emit(bound, a.scales);
+    if (!a.norms2) return;
+    v = 0.0f;
+    for (uint32_t c = threadIdx.x; c < a.channels; c += 256) v = fmaxf(v, fabsf(a.bias2[c]) + a.norms2[c] * bound);
+    emit(block_max_256(v, red), a.scales + 2);
+}
+
+// f32 [image][channel][h][w] to the halves layout, border included: a thread
+// per word pair (both terms), channels in groups of eight.
+__global__ __launch_bounds__(256) void to_halves_kernel(const float *in, uint32_t channels, uint32_t h, uint32_t w,
+                                                        const float *scales, uint8_t *out) {
+    const HalvesPlane p = halves_plane(h, w);
+    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= p.words) return;
+    const uint32_t c0 = blockIdx.y * 8, b = blockIdx.z;
+    const uint32_t row = i / (2 * p.slots), rest = i % (2 * p.slots);
+    const uint32_t col = 2 * (rest % p.slots) + rest / p.slots;
+    const bool inside = row >= 1 && row <= h && col >= 1 && col <= w;
+    const float up = scales[0];
+    const float *src = in + (((size_t)b * channels + c0) * h + (inside ? row - 1 : 0)) * w + (inside ? col - 1 : 0);
+    ch8 hi, lo;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+        _Float16 x, y;
+        split_half(inside ? src[(size_t)k * h * w] : 0.0f, up, x, y);
+        hi[k] = x, lo[k] = y;
+    }
+    uint8_t *to = out + ((((size_t)b * (channels / kMfIc) + c0 / kMfIc) * 4 + (c0 / 8 & 1)) * p.words + i) * 16;
+    *reinterpret_cast<ch8 *>(to) = hi;
+    *reinterpret_cast<ch8 *>(to + (size_t)2 * p.words * 16) = lo;
+}
+
+// conv1 of the tower (one input channel) from the log-mel [bins][frames]
+// straight to the halves layout: image b is the chunk_frames frames from
+// chunk first + b (zero past the clip, model.zig:557-563). A thread takes one
+// word position of the padded output plane and 16 channels: its nine samples
+// are read once, each output is bias + the taps in the reference's order, then
+// GELU and the two terms; border words are zero.
+struct Conv1HalvesArgs {
+    const float *mel;
+    const uint16_t *weights;
+    const float *bias, *scales;
+    uint8_t *out;
+    uint32_t bins, frames, chunk_frames, first, channels, oh, ow;
+};
+
+__global__ __launch_bounds__(256) void conv1_halves_kernel(const Conv1HalvesArgs a) {
+    __shared__ float wts[kMfIc][9];
+    __shared__ float bs[kMfIc];
+    const uint32_t c0 = blockIdx.y * kMfIc, b = blockIdx.z;
+    if (threadIdx.x < kMfIc * 9)
+        wts[threadIdx.x / 9][threadIdx.x % 9] = dev::f16_bits_to_f32(a.weights[(size_t)c0 * 9 + threadIdx.x]);
+    if (threadIdx.x < kMfIc) bs[threadIdx.x] = a.bias[c0 + threadIdx.x];
+    __syncthreads();
+    const HalvesPlane p = halves_plane(a.oh, a.ow);
+    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= p.words) return;
+    const uint32_t prow = i / (2 * p.slots), rest = i % (2 * p.slots);
+    const uint32_t pcol = 2 * (rest % p.slots) + rest / p.slots;
+    cu4 *to = reinterpret_cast<cu4 *>(a.out) + ((size_t)b * (a.channels / kMfIc) + blockIdx.y) * 4 * p.words + i;
+    if (prow < 1 || prow > a.oh || pcol < 1 || pcol > a.ow) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) to[(size_t)k * p.words] = cu4{0, 0, 0, 0};
+        return;
+    }
+    const uint64_t frame0 = (uint64_t)(a.first + b) * a.chunk_frames;
+    float x[9];
+    bool ok[9];
+#pragma unroll
+    for (int tap = 0; tap < 9; ++tap) {
+        const int r = (int)(prow - 1) * 2 + tap / 3 - 1, c = (int)(pcol - 1) * 2 + tap % 3 - 1;
+        ok[tap] = r >= 0 && r < (int)a.bins && c >= 0 && c < (int)a.chunk_frames;
+        x[tap] = ok[tap] && frame0 + c < a.frames ? a.mel[(size_t)r * a.frames + frame0 + c] : 0.0f;
+    }
+    const float up = a.scales[0];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        ch8 hi, lo;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            float acc = 0.0f;
+#pragma unroll
+            for (int tap = 0; tap < 9; ++tap)
+                if (ok[tap]) acc = fmaf(wts[8 * h + k][tap], x[tap], acc);
+            _Float16 u, l;
+            split_half(dev::gelu(bs[8 * h + k] + acc), up, u, l);
+            hi[k] = u, lo[k] = l;
+        }
+        to[(size_t)h * p.words] = __builtin_bit_cast(cu4, hi);
+        to[(size_t)(2 + h) * p.words] = __builtin_bit_cast(cu4, lo);
     }
 }
 
@@ -421,51 +655,219 @@ hipError_t launch_conv3x3s2_gelu(hipStream_t s, float *out, const float *in, con
 
 namespace {
 
-// Patch rows for kMfPos positions starting anywhere in a row of `ow`.
-uint32_t mfma_patch_rows(uint32_t ow) { return 2 * ((kMfPos - 1 + ow - 1) / ow) + 3; }
+// Patch rows for `positions` positions starting anywhere in a row of `ow`.
+uint32_t mfma_patch_rows(uint32_t ow, uint32_t positions = kMfPos) { return 2 * ((positions - 1 + ow - 1) / ow) + 3; }
+
+uint32_t mfma_oc_pad(uint32_t out_ch) { return (out_ch + 63) / 64 * 64; }
+
+constexpr uint32_t kMaximaBlocks = 256;
+
+// Workspace pieces of a prepared convolution: operand-order weights, channel
+// sums, partial maxima and scales, 256-byte aligned.
+size_t piece(size_t bytes) { return (bytes + 255) & ~(size_t)255; }
+size_t wprep_bytes(uint32_t out_ch, uint32_t in_ch) { return piece((size_t)mfma_oc_pad(out_ch) * in_ch * 9 * 2); }
+size_t norms_bytes(uint32_t out_ch) { return piece((size_t)mfma_oc_pad(out_ch) * sizeof(float)); }
+constexpr size_t kMaximaBytes = kMaximaBlocks * sizeof(float);
+constexpr size_t kScaleBytes = 256;
+
+size_t halves_image_bytes(uint32_t channels, uint32_t h, uint32_t w) {
+    return (size_t)channels / kMfIc * 4 * halves_plane(h, w).words * 16;
+}
+
+template <int NT, bool HALVES>
+hipError_t launch_mfma_tiles(hipStream_t s, ConvMfmaArgs a, uint32_t batch) {
+    const HalvesPlane p = halves_plane(a.h, a.w);
+    a.patch_rows = std::min(mfma_patch_rows(a.ow, 32 * NT), a.h + 2);
+    a.pos_tiles = (a.positions + 32 * NT - 1) / (32 * NT);
+    a.units = batch * a.pos_tiles;
+    a.oc_blocks = (a.out_ch + kMfOc - 1) / kMfOc;
+    const uint32_t grid = (a.units + 7) / 8 * 8 * a.oc_blocks;
+    const uint32_t rounds = (a.patch_rows * 2 * p.slots * 4 + 255) / 256;
+    if (rounds <= 2) conv3x3s2_gelu_mfma_kernel<NT, 2, HALVES><<<grid, 256, 0, s>>>(a);
+    else if (rounds <= 4) conv3x3s2_gelu_mfma_kernel<NT, 4, HALVES><<<grid, 256, 0, s>>>(a);
+    else if (rounds <= 6) conv3x3s2_gelu_mfma_kernel<NT, 6, HALVES><<<grid, 256, 0, s>>>(a);
+    else if (rounds <= 8) conv3x3s2_gelu_mfma_kernel<NT, 8, HALVES><<<grid, 256, 0, s>>>(a);
+    else if (rounds <= kMfRounds) conv3x3s2_gelu_mfma_kernel<NT, kMfRounds, HALVES><<<grid, 256, 0, s>>>(a);
+    else return hipErrorInvalidValue;
+    return hipGetLastError();
+}
+
+// 32-position workgroups where 64-position ones leave compute units idle or
+// unevenly filled: a compute unit's share took about 42 us a workgroup of 32
+// positions and 63 of 64 (30 stages; 30 s of audio conv3 89 / 82 us, conv2 253
+// / 252; 4 s conv2 54 / 78, conv3 40 / 66; 11 s conv2 122 / 131).
+template <bool HALVES>
+hipError_t launch_mfma(hipStream_t s, int cus, const ConvMfmaArgs &a, uint32_t batch) {
+    auto share = [&](uint32_t positions) {
+        const uint64_t groups = (uint64_t)batch * ((a.positions + positions - 1) / positions) *
+                                ((a.out_ch + kMfOc - 1) / kMfOc);
+        return (groups + (uint32_t)cus - 1) / (uint32_t)cus;
+    };
+    return 2 * share(32) <= 3 * share(64) ? launch_mfma_tiles<1, HALVES>(s, a, batch)
+                                          : launch_mfma_tiles<2, HALVES>(s, a, batch);
+}
+
+ConvMfmaArgs mfma_args(const void *in, const void *wprep, const float *bias, const float *scales, uint32_t out_ch,
+                       uint32_t in_ch, uint32_t h, uint32_t w) {
+    ConvMfmaArgs a{};
+    a.in = static_cast<const uint8_t *>(in);
+    a.wprep = static_cast<const uint8_t *>(wprep);
+    a.bias = bias;
+    a.scales = scales;
+    a.out_ch = out_ch;
+    a.oc_tiles = mfma_oc_pad(out_ch) / 32;
+    a.stages = in_ch / kMfIc;
+    a.h = h, a.w = w;
+    a.oh = (h - 1) / 2 + 1, a.ow = (w - 1) / 2 + 1;
+    a.positions = a.oh * a.ow;
+    return a;
+}
 
 }  // namespace
-
-size_t conv_mfma_prep_bytes(uint32_t out_ch, uint32_t in_ch) {
-    const uint32_t oc_pad = (out_ch + kMfOc - 1) / kMfOc * kMfOc;
-    return (size_t)oc_pad * in_ch * 9 * 2 * sizeof(uint16_t);
-}
 
 bool conv_mfma_supported(uint32_t in_ch, uint32_t h, uint32_t w) {
     if (in_ch == 0 || in_ch % kMfIc || h == 0 || w == 0) return false;
     const uint32_t ow = (w - 1) / 2 + 1;
-    const uint64_t cells = (uint64_t)mfma_patch_rows(ow) * (w + 2);
-    // Two channel halves per cell in kMfRounds rounds of 256 threads; two
-    // buffers of two terms in LDS.
-    return 2 * cells <= 256u * kMfRounds && cells * kMfIcPad * 2 * 2 * sizeof(uint16_t) <= kMfLdsMax;
+    // Four planes of patch words, kMfRounds of 256, in each of two LDS buffers.
+    return (uint64_t)mfma_patch_rows(ow) * 2 * ((w + 3) / 2) * 4 <= 256u * kMfRounds;
 }
 
-hipError_t launch_conv_mfma_prep(hipStream_t s, const uint16_t *weights, uint32_t out_ch, uint32_t in_ch, void *wprep) {
-    const uint32_t oc_pad = (out_ch + kMfOc - 1) / kMfOc * kMfOc;
-    conv_mfma_prep_kernel<<<blocks_for((uint64_t)oc_pad * in_ch * 9), 256, 0, s>>>(weights, out_ch, oc_pad, in_ch,
-                                                                                   static_cast<uint16_t *>(wprep));
-    return hipGetLastError();
+// One convolution over f32 planes: images of at most this many bytes of
+// activation terms at a time (at least one).
+constexpr size_t kConvGroupBytes = (size_t)256 << 20;
+
+uint32_t conv_mfma_group(uint32_t batch, uint32_t in_ch, uint32_t h, uint32_t w) {
+    const size_t image = halves_image_bytes(in_ch, h, w);
+    return (uint32_t)std::min<size_t>(batch, std::max<size_t>(1, kConvGroupBytes / image));
 }
 
-hipError_t launch_conv3x3s2_gelu_mfma(hipStream_t s, float *out, const float *in, const void *wprep, const float *bias,
-                                     uint32_t batch, uint32_t out_ch, uint32_t in_ch, uint32_t h, uint32_t w) {
+size_t conv_mfma_bytes(uint32_t batch, uint32_t out_ch, uint32_t in_ch, uint32_t h, uint32_t w) {
+    return wprep_bytes(out_ch, in_ch) + norms_bytes(out_ch) + kMaximaBytes + kScaleBytes +
+           conv_mfma_group(batch, in_ch, h, w) * halves_image_bytes(in_ch, h, w);
+}
+
+hipError_t launch_conv3x3s2_gelu_mfma(hipStream_t s, int cus, float *out, const float *in, const uint16_t *weights,
+                                      const float *bias, uint32_t batch, uint32_t out_ch, uint32_t in_ch, uint32_t h,
+                                      uint32_t w, void *scratch) {
     if (!conv_mfma_supported(in_ch, h, w) || batch == 0 || batch > 65535) return hipErrorInvalidValue;
-    ConvMfmaArgs a{};
-    a.out = out, a.in = in, a.wprep = static_cast<const uint16_t *>(wprep), a.bias = bias;
-    a.out_ch = out_ch, a.oc_pad = (out_ch + kMfOc - 1) / kMfOc * kMfOc, a.in_ch = in_ch, a.h = h, a.w = w;
-    a.oh = (h - 1) / 2 + 1, a.ow = (w - 1) / 2 + 1;
-    a.positions = a.oh * a.ow;
-    a.patch_rows = mfma_patch_rows(a.ow);
-    a.patch_cols = w + 2;
-    const size_t lds = (size_t)a.patch_rows * a.patch_cols * kMfIcPad * 2 * 2 * sizeof(uint16_t);
-    // (Above the default 64 KB of dynamic LDS: raised once, to the most any
-    // supported shape asks for.)
-    static const hipError_t raised = hipFuncSetAttribute(reinterpret_cast<const void *>(&conv3x3s2_gelu_mfma_kernel),
-                                                         hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMfLdsMax);
-    if (raised != hipSuccess) return raised;
-    const dim3 grid(a.oc_pad / kMfOc, (a.positions + kMfPos - 1) / kMfPos, batch);
-    conv3x3s2_gelu_mfma_kernel<<<grid, 256, lds, s>>>(a);
+    uint8_t *at = static_cast<uint8_t *>(scratch);
+    uint8_t *wprep = at;
+    float *norms = reinterpret_cast<float *>(at += wprep_bytes(out_ch, in_ch));
+    float *partial = reinterpret_cast<float *>(at += norms_bytes(out_ch));
+    float *scales = reinterpret_cast<float *>(at += kMaximaBytes);
+    uint8_t *halves = at + kScaleBytes;
+    ConvPrepArgs p{};
+    p.job[0] = {weights, wprep, norms, out_ch, mfma_oc_pad(out_ch), in_ch};
+    p.x = in;
+    p.count = (uint64_t)batch * in_ch * h * w;
+    p.partial = partial;
+    p.partials = (uint32_t)std::min<uint64_t>(kMaximaBlocks, (p.count + 255) / 256);
+    conv_prep_kernel<<<p.job[0].oc_pad + p.partials, 256, 0, s>>>(p);
+    ConvScaleArgs c{};
+    c.partial = partial;
+    c.partials = p.partials;
+    c.scales = scales;
+    conv_scale_kernel<<<1, 256, 0, s>>>(c);
+    ConvMfmaArgs a = mfma_args(halves, wprep, bias, scales, out_ch, in_ch, h, w);
+    const uint32_t group = conv_mfma_group(batch, in_ch, h, w);
+    for (uint32_t b = 0; b < batch; b += group) {
+        const uint32_t n = std::min(group, batch - b);
+        to_halves_kernel<<<dim3((halves_plane(h, w).words + 255) / 256, in_ch / 8, n), 256, 0, s>>>(
+            in + (size_t)b * in_ch * h * w, in_ch, h, w, scales, halves);
+        a.out = out + (size_t)b * out_ch * a.positions;
+        const hipError_t e = launch_mfma<false>(s, cus, a, n);
+        if (e != hipSuccess) return e;
+    }
     return hipGetLastError();
+}
+
+// The tower's three convolutions with conv2 and conv3 in this form.
+namespace {
+
+struct TowerPieces {
+    size_t wprep2, wprep3, norms2, norms3, partial, scales, halves1, halves2, total;
+};
+
+TowerPieces tower_pieces(const ConvTower &c) {
+    const uint32_t h1 = (c.bins - 1) / 2 + 1, w1 = (c.chunk_frames - 1) / 2 + 1;
+    const uint32_t h2 = (h1 - 1) / 2 + 1, w2 = (w1 - 1) / 2 + 1;
+    TowerPieces p{};
+    size_t at = 0;
+    auto take = [&](size_t bytes) {
+        const size_t here = at;
+        at += bytes;
+        return here;
+    };
+    p.wprep2 = take(wprep_bytes(c.channels, c.channels));
+    p.wprep3 = take(wprep_bytes(c.channels, c.channels));
+    p.norms2 = take(norms_bytes(c.channels));
+    p.norms3 = take(norms_bytes(c.channels));
+    p.partial = take(kMaximaBytes);
+    p.scales = take(kScaleBytes);
+    p.halves1 = take(piece(c.group * halves_image_bytes(c.channels, h1, w1)));
+    p.halves2 = take(piece(c.group * halves_image_bytes(c.channels, h2, w2)));
+    p.total = at;
+    return p;
+}
+
+}  // namespace
+
+bool conv_tower_supported(const ConvTower &c) {
+    const uint32_t h1 = (c.bins - 1) / 2 + 1, w1 = (c.chunk_frames - 1) / 2 + 1;
+    const uint32_t h2 = (h1 - 1) / 2 + 1, w2 = (w1 - 1) / 2 + 1;
+    return conv_mfma_supported(c.channels, h1, w1) && conv_mfma_supported(c.channels, h2, w2);
+}
+
+size_t conv_tower_bytes(const ConvTower &c) { return tower_pieces(c).total; }
+
+hipError_t launch_conv_tower_prep(hipStream_t s, const ConvTower &c, const float *mel, uint32_t frames, void *scratch) {
+    uint8_t *base = static_cast<uint8_t *>(scratch);
+    const TowerPieces at = tower_pieces(c);
+    const uint32_t pad = mfma_oc_pad(c.channels);
+    ConvPrepArgs p{};
+    p.job[0] = {c.weights[1], base + at.wprep2, reinterpret_cast<float *>(base + at.norms2), c.channels, pad, c.channels};
+    p.job[1] = {c.weights[2], base + at.wprep3, reinterpret_cast<float *>(base + at.norms3), c.channels, pad, c.channels};
+    p.x = mel;
+    p.count = (uint64_t)c.bins * frames;
+    p.partial = reinterpret_cast<float *>(base + at.partial);
+    p.partials = (uint32_t)std::min<uint64_t>(kMaximaBlocks, (p.count + 255) / 256);
+    conv_prep_kernel<<<2 * pad + p.partials, 256, 0, s>>>(p);
+    ConvScaleArgs q{};
+    q.partial = p.partial;
+    q.partials = p.partials;
+    q.conv1 = c.weights[0];
+    q.bias1 = c.bias[0];
+    q.norms2 = p.job[0].norms;
+    q.bias2 = c.bias[1];
+    q.channels = c.channels;
+    q.scales = reinterpret_cast<float *>(base + at.scales);
+    conv_scale_kernel<<<1, 256, 0, s>>>(q);
+    return hipGetLastError();
+}
+
+hipError_t launch_conv_tower(hipStream_t s, int cus, const ConvTower &c, const float *mel, uint32_t frames, uint32_t first,
+                             uint32_t count, float *out, void *scratch) {
+    uint8_t *base = static_cast<uint8_t *>(scratch);
+    const TowerPieces at = tower_pieces(c);
+    const float *scales = reinterpret_cast<const float *>(base + at.scales);
+    const uint32_t h1 = (c.bins - 1) / 2 + 1, w1 = (c.chunk_frames - 1) / 2 + 1;
+    Conv1HalvesArgs k{};
+    k.mel = mel;
+    k.weights = c.weights[0];
+    k.bias = c.bias[0];
+    k.scales = scales;
+    k.out = base + at.halves1;
+    k.bins = c.bins, k.frames = frames, k.chunk_frames = c.chunk_frames, k.first = first, k.channels = c.channels;
+    k.oh = h1, k.ow = w1;
+    conv1_halves_kernel<<<dim3((halves_plane(h1, w1).words + 255) / 256, c.channels / kMfIc, count), 256, 0, s>>>(k);
+    ConvMfmaArgs a = mfma_args(base + at.halves1, base + at.wprep2, c.bias[1], scales, c.channels, c.channels, h1, w1);
+    a.halves = base + at.halves2;
+    const hipError_t e = launch_mfma<true>(s, cus, a, count);
+    if (e != hipSuccess) return e;
+    ConvMfmaArgs a3 = mfma_args(base + at.halves2, base + at.wprep3, c.bias[2], scales + 2, c.channels, c.channels, a.oh,
+                                a.ow);
+    a3.out = out;
+    return launch_mfma<false>(s, cus, a3, count);
 }
 
 hipError_t launch_gather_chunks(hipStream_t s, const float *mel, uint32_t bins, uint32_t frames, uint32_t chunk_frames,
