@@ -996,8 +996,13 @@ int32_t qwh_decoder_create_cache(qwh_ctx *ctx, const qwh_decoder_config *config,
     build_rope_tables(cos_t, sin_t, half, c.theta, c.max_positions);
     if (st == QWH_OK) st = dalloc(d, cos_t.size() * 4, reinterpret_cast<void **>(&d->rope_cos));
     if (st == QWH_OK) st = dalloc(d, sin_t.size() * 4, reinterpret_cast<void **>(&d->rope_sin));
-    if (st == QWH_OK) st = check_hip(ctx, hipMemcpy(d->rope_cos, cos_t.data(), cos_t.size() * 4, hipMemcpyHostToDevice), "rope");
-    if (st == QWH_OK) st = check_hip(ctx, hipMemcpy(d->rope_sin, sin_t.data(), sin_t.size() * 4, hipMemcpyHostToDevice), "rope");
+    // (On the context's stream, after dalloc's zeros: the default stream does
+    // not wait for them. The host tables must outlive the copies.)
+    if (st == QWH_OK)
+        st = check_hip(ctx, hipMemcpyAsync(d->rope_cos, cos_t.data(), cos_t.size() * 4, hipMemcpyHostToDevice, ctx->stream), "rope");
+    if (st == QWH_OK)
+        st = check_hip(ctx, hipMemcpyAsync(d->rope_sin, sin_t.data(), sin_t.size() * 4, hipMemcpyHostToDevice, ctx->stream), "rope");
+    if (hipStreamSynchronize(ctx->stream) != hipSuccess && st == QWH_OK) st = check_hip(ctx, hipGetLastError(), "rope");
     // Caches: per sequence, per layer [scales][codes] (decoder.zig:58-65),
     // or [max_positions][kv_width] f32 (decoder.zig:77-83).
     if (cache_format == QWH_CACHE_Q8) {
