@@ -231,20 +231,23 @@ __device__ __forceinline__ void rows_block(const RowsArgs &a, uint32_t row_block
             __builtin_memcpy(cs, &v, 2 * CG);
         }
     };
-    // Group gc + i of the chunk taken at gc.
-    auto step = [&](auto at, uint32_t gc) __attribute__((always_inline)) {
+    // Group gc + i of the chunk taken at gc; `tail`: of the last, shorter chunk.
+    auto step = [&](auto at, auto tail, uint32_t gc) __attribute__((always_inline)) {
         constexpr int i = decltype(at)::value;
+        constexpr bool ahead = !decltype(tail)::value;
         const uint32_t g = gc + i;
         // This group's words have landed (what was issued after them, the
         // next group's and in some steps a chunk of weights, may still be on
         // its way: vector memory completes in order), in every wavefront
         // after the barrier; the buffer refilled now was last read before it.
-        constexpr int after = PT + ((i == 1 || i == 2 || CG == 2) ? WL : 0);
+        // No weights follow the last chunk (the compiler would drop loads that
+        // nothing uses, and a count that expects them would not wait).
+        constexpr int after = PT + (ahead && (i == 1 || i == 2 || CG == 2) ? WL : 0);
         __builtin_amdgcn_s_waitcnt(kWait<after>);
         __builtin_amdgcn_s_barrier();
         load_acts(min(g + 2, g1 - 1), buf == 0 ? 2 : buf - 1);
         __builtin_amdgcn_sched_barrier(0);
-        if constexpr (i == 0) {
+        if constexpr (i == 0 && ahead) {
             // The next chunk's weights travel while this one multiplies.
             load_weights(min(gc + CG, g1 - 1));
             __builtin_amdgcn_sched_barrier(0);
@@ -275,12 +278,12 @@ __device__ __forceinline__ void rows_block(const RowsArgs &a, uint32_t row_block
     uint32_t gc = g0;
     for (; gc + CG <= g1; gc += CG) {
         take_chunk(gc);
-        static_for<CG>([&](auto at) __attribute__((always_inline)) { step(at, gc); });
+        static_for<CG>([&](auto at) __attribute__((always_inline)) { step(at, std::false_type{}, gc); });
     }
     if (gc < g1) {
         take_chunk(gc);
         static_for<CG>([&](auto at) __attribute__((always_inline)) {
-            if (gc + decltype(at)::value < g1) step(at, gc);
+            if (gc + decltype(at)::value < g1) step(at, std::true_type{}, gc);
         });
     }
 
