@@ -62,10 +62,18 @@ __device__ __forceinline__ float wave_sum(float v) {
 }
 
 // The reference's erf (math.zig:46-60): the Numerical Recipes Chebyshev fit
-// of erfc (`erfcc`), evaluated in f32 by Horner's rule.
+// of erfc (`erfcc`), evaluated in f32 by Horner's rule. Its reciprocal is the
+// hardware's refined by one Newton step and its exponential the hardware's
+// exp2 of the scaled argument with the scaling's rounding put back, both
+// within an ulp: half the instructions of the library's division and expf
+// (conv1 of the front end, 46M values, 97 -> 82 us; the error against 64 bits
+// is the same, 4.5e-7 at most). |x| past 16 is saturated
+// as it is at 16 (exp(-256) is 0).
 __device__ __forceinline__ float erf_fit(float x) {
-    const float magnitude = fabsf(x);
-    const float t = 1.0f / (1.0f + 0.5f * magnitude);
+    const float magnitude = fminf(fabsf(x), 16.0f);
+    const float d = 1.0f + 0.5f * magnitude;
+    const float r = __builtin_amdgcn_rcpf(d);
+    const float t = fmaf(fmaf(-d, r, 1.0f), r, r);
     float poly = -0.82215223f + t * 0.17087277f;
     poly = 1.48851587f + t * poly;
     poly = -1.13520398f + t * poly;
@@ -74,7 +82,13 @@ __device__ __forceinline__ float erf_fit(float x) {
     poly = 0.09678418f + t * poly;
     poly = 0.37409196f + t * poly;
     poly = 1.00002368f + t * poly;
-    const float tau = t * expf(-magnitude * magnitude - 1.26551223f + t * poly);
+    const float y = -magnitude * magnitude - 1.26551223f + t * poly;
+    const float log2e = 1.44269504f, ln2 = 0.693147181f;
+    const float h = y * log2e;
+    // y log2(e) = h + its rounding + y times the constant's.
+    const float l = fmaf(y, log2e, -h) + y * 1.92596299e-8f;
+    const float e = __builtin_amdgcn_exp2f(h);
+    const float tau = t * fmaf(e, l * ln2, e);
     return copysignf(1.0f - tau, x);
 }
 
