@@ -742,9 +742,9 @@ __global__ __launch_bounds__(64 * W) void gemm_f16_kernel(const DenseArgs a) {
 // token l % 16, so the epilogue needs no cross-wavefront sum: residual,
 // siluMul of gate / up pairs (rows 2p, 2p + 1 sit in the same lane), or
 // RMSNorm's inverse RMS per token.
-template <bool Norm, int R, int T, int W>
+template <bool Norm, int R, int T, int W, int C>
 __global__ __launch_bounds__(64 * W) void gemm_f16_rows_kernel(const DenseArgs a) {
-    constexpr int C = 2;                      // steps per chunk, and steps of weight loads in flight
+    // C: steps per chunk, and steps of weight loads in flight.
     constexpr int kUnits = C * T;             // staging units per chunk: [tile][step]
     constexpr int kGroups = W / 2;            // 128-thread staging groups
     constexpr int NU = kUnits / kGroups;      // units per thread per chunk
@@ -946,12 +946,11 @@ __global__ __launch_bounds__(64 * W) void gemm_f16_rows_kernel(const DenseArgs a
     }
 }
 
-template <bool Norm, int R, int T, int W>
+template <bool Norm, int R, int T, int W, int C>
 hipError_t launch_f16_rows(hipStream_t s, uint32_t tokens, const DenseArgs &a) {
-    constexpr int C = 2;
     const dim3 grid((a.rows + 16 * R * W - 1) / (16 * R * W), (tokens + 16 * T - 1) / (16 * T));
     const size_t lds = (Norm ? (size_t)a.cols * 4 : 0) + 2 * ((size_t)C * T * 4 * 64 * 16 + (size_t)C * T * 16 * 4);
-    void (*kernel)(const DenseArgs) = gemm_f16_rows_kernel<Norm, R, T, W>;
+    void (*kernel)(const DenseArgs) = gemm_f16_rows_kernel<Norm, R, T, W, C>;
     if (lds > (48u << 10)) {
         const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
                                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
@@ -984,8 +983,8 @@ constexpr size_t kMaxWorkgroupLds = 160u << 10;  // gfx950
 // LDS of the f16 forms apart from RMSNorm weights: the rows form's two
 // operand buffers and its per-group squares; the K-split form's
 // activation tiles, partial tiles and squares (four wavefronts).
-constexpr size_t rows_form_lds(int t, int w) {
-    return 2 * ((size_t)2 * t * 4 * 64 * 16 + (size_t)2 * t * 16 * 4) + (size_t)(w / 2) * t * 16 * 4;
+constexpr size_t rows_form_lds(int t, int w, int c) {
+    return 2 * ((size_t)c * t * 4 * 64 * 16 + (size_t)c * t * 16 * 4) + (size_t)(w / 2) * t * 16 * 4;
 }
 constexpr size_t ksplit_form_lds(int r) { return (size_t)4 * 16 * 17 * 16 + (size_t)4 * 16 * r * 17 * 4 + 4 * 16 * 4; }
 
@@ -1012,6 +1011,64 @@ hipError_t launch_f16_mma(hipStream_t s, uint32_t tokens, size_t lds, const Dens
     }
     hipLaunchKernelGGL(kernel, grid, dim3(64 * W), lds, s, a);
     return hipGetLastError();
+}
+
+template <bool Norm, int R>
+hipError_t launch_f16_ksplit(hipStream_t s, uint32_t tokens, const DenseArgs &a) {
+    return launch_f16_mma<Norm, R, 4, 2>(s, tokens, Norm ? (size_t)a.cols * 4 : 0, a);
+}
+
+// The f16 forms for more than 16 tokens: rows x tokens of a workgroup, its
+// LDS, and its time in us -- fixed + step * (K / 64) while every CU has at
+// most one, `round` of that for each workgroup a CU runs where some have more
+// -- as a sweep over 1024 x 1024 to 151936 x 2048 at 17 to 402 tokens measured
+// them (within 15 %). The K-split forms have the shortest chain of steps and
+// fill the device with few rows and tokens; the others read the weights, and
+// split the activations, less often. Before, rows alone chose among the rows
+// forms: 4096 x 2048 at 37 tokens 24.9 us, now 13.5; 1024 x 3072 29.6 and 8.5;
+// 2048 x 6144 58 and 22.4; 12288 x 2048 at 17 tokens 26.3 and 18.8, at 128
+// 54.7 and 37.4.
+struct F16Form {
+    uint32_t rows, tokens;
+    size_t lds;
+    float fixed, step, round;
+    hipError_t (*plain)(hipStream_t, uint32_t, const DenseArgs &);
+    hipError_t (*normed)(hipStream_t, uint32_t, const DenseArgs &);
+};
+
+template <int R>
+constexpr F16Form ksplit_form(float fixed, float step, float round) {
+    return {16 * R, 16, ksplit_form_lds(R), fixed, step, round, launch_f16_ksplit<false, R>, launch_f16_ksplit<true, R>};
+}
+
+template <int R, int T, int W, int C>
+constexpr F16Form rows_form(float fixed, float step, float round) {
+    return {16 * R * W, 16 * T, rows_form_lds(T, W, C), fixed, step, round, launch_f16_rows<false, R, T, W, C>,
+            launch_f16_rows<true, R, T, W, C>};
+}
+
+// The form with the least estimated time whose LDS (`norm_lds` bytes of
+// RMSNorm weights beside it) fits a workgroup; null if none does.
+const F16Form *f16_form(int cus, uint32_t rows, uint32_t cols, uint32_t tokens, size_t norm_lds) {
+    static constexpr F16Form forms[] = {
+        ksplit_form<1>(2.0f, 0.150f, 0.80f),        ksplit_form<2>(2.2f, 0.215f, 0.86f),
+        ksplit_form<3>(2.6f, 0.335f, 0.94f),        ksplit_form<4>(2.2f, 0.355f, 0.83f),
+        rows_form<1, 2, 4, 4>(3.1f, 0.445f, 0.82f), rows_form<1, 3, 4, 4>(4.7f, 0.540f, 0.96f),
+        rows_form<1, 2, 8, 2>(2.6f, 0.725f, 1.00f), rows_form<1, 4, 8, 2>(5.0f, 0.945f, 0.95f),
+        rows_form<2, 4, 8, 2>(6.5f, 1.420f, 1.15f),
+    };
+    const uint64_t cu = (uint64_t)(cus > 0 ? cus : 256);
+    const F16Form *best = nullptr;
+    float least = 0.0f;
+    for (const F16Form &f : forms) {
+        if (norm_lds + f.lds > kMaxWorkgroupLds) continue;
+        const uint64_t groups = (uint64_t)((rows + f.rows - 1) / f.rows) * ((tokens + f.tokens - 1) / f.tokens);
+        const uint64_t rounds = (groups + cu - 1) / cu;
+        float us = f.fixed + f.step * (float)(cols / 64);
+        if (rounds > 1) us *= f.round * (float)rounds;
+        if (!best || us < least) best = &f, least = us;
+    }
+    return best;
 }
 
 // f16 bits of each value, round to nearest even (half_float.zig:12-16).
@@ -1062,24 +1119,10 @@ hipError_t launch_gemv_dense(hipStream_t s, int cus, const GemvInput &in, const 
             // fits a workgroup's 160 KiB.
             const size_t norm_lds = norm ? (size_t)w.cols * 4 : 0;
             auto fits = [&](size_t bytes) { return norm_lds + bytes <= kMaxWorkgroupLds; };
-            // More than 16 tokens: the rows form, T token tiles sharing each
-            // weight load (measured best on the 1.7B shapes at 32 to 256
-            // tokens and the lm_head at 64).
-            if (tokens > 16) {
-                if (w.rows < 8192) {
-                    if (w.rows >= 4096 && fits(rows_form_lds(2, 8)))
-                        return norm ? launch_f16_rows<true, 1, 2, 8>(s, tokens, a) : launch_f16_rows<false, 1, 2, 8>(s, tokens, a);
-                    if (w.rows < 4096 && fits(rows_form_lds(2, 4)))
-                        return norm ? launch_f16_rows<true, 1, 2, 4>(s, tokens, a) : launch_f16_rows<false, 1, 2, 4>(s, tokens, a);
-                } else if (tokens >= 128 && fits(rows_form_lds(4, 8))) {
-                    return norm ? launch_f16_rows<true, 2, 4, 8>(s, tokens, a) : launch_f16_rows<false, 2, 4, 8>(s, tokens, a);
-                } else if (tokens < 128 && w.rows >= 65536 && fits(rows_form_lds(4, 8))) {
-                    return norm ? launch_f16_rows<true, 1, 4, 8>(s, tokens, a) : launch_f16_rows<false, 1, 4, 8>(s, tokens, a);
-                } else if (tokens < 128 && w.rows < 65536 && fits(rows_form_lds(2, 8))) {
-                    return norm ? launch_f16_rows<true, 1, 2, 8>(s, tokens, a) : launch_f16_rows<false, 1, 2, 8>(s, tokens, a);
-                }
-            }
-            // Up to 16 tokens (or rows-form LDS too large): K split over the
+            if (tokens > 16)
+                if (const F16Form *form = f16_form(cus, w.rows, w.cols, tokens, norm_lds))
+                    return norm ? form->normed(s, tokens, a) : form->plain(s, tokens, a);
+            // Up to 16 tokens (or no form's LDS fits): K split over the
             // wavefronts, R row tiles per workgroup from the 16 x 16 tiles
             // per CU: up to 3, one workgroup per CU with that many (each
             // activation step then loaded once per CU: gate|up at 16 tokens
