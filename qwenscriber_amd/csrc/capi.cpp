@@ -1103,7 +1103,7 @@ int32_t qwh_conv3x3s2_gelu(qwh_ctx *ctx, float *out_dev, const float *in_dev, co
     if (conv_mfma_supported(in_channels, in_height, in_width)) {
         // The matrix-core form, its weights and activation terms prepared in
         // the context's scratch.
-        QWH_TRY(ensure_workspace(ctx, ctx->scratch, conv_mfma_bytes(batch, out_channels, in_channels, in_height, in_width)));
+        QWH_TRY(ensure_workspace(ctx, ctx->scratch, conv_mfma_bytes(ctx->cus, batch, out_channels, in_channels, in_height, in_width)));
         return check_hip(ctx, launch_conv3x3s2_gelu_mfma(ctx->stream, ctx->cus, out_dev, in_dev, weights_dev, bias_dev, batch,
                                                          out_channels, in_channels, in_height, in_width,
                                                          ctx->scratch.ptr),
@@ -1174,14 +1174,14 @@ int32_t qwh_audio_frontend(qwh_ctx *ctx, const qwh_audio_frontend_weights *w, co
     const size_t off_flat = off3 + align(group * p3);
     const size_t off_tower = off_flat + align((size_t)group * chunk_steps * features);
     const bool mfma2 = conv_mfma_supported(downsample, h1, w1), mfma3 = conv_mfma_supported(downsample, h2, w2);
-    const size_t tower_bytes = fused ? conv_tower_bytes(tower)
-                                     : std::max(mfma2 ? conv_mfma_bytes(group, downsample, downsample, h1, w1) : 0,
-                                                mfma3 ? conv_mfma_bytes(group, downsample, downsample, h2, w2) : 0);
+    const size_t tower_bytes = fused ? conv_tower_bytes(ctx->cus, tower)
+                                     : std::max(mfma2 ? conv_mfma_bytes(ctx->cus, group, downsample, downsample, h1, w1) : 0,
+                                                mfma3 ? conv_mfma_bytes(ctx->cus, group, downsample, downsample, h2, w2) : 0);
     const size_t total = off_tower + align(tower_bytes / sizeof(float) + 1);
     QWH_TRY(ensure_workspace(ctx, ctx->front, total * sizeof(float)));
     float *ws = static_cast<float *>(ctx->front.ptr);
     hipStream_t s = ctx->stream;
-    if (fused) QWH_TRY(check_hip(ctx, launch_conv_tower_prep(s, tower, log_mel_dev, frames, ws + off_tower), "front-end prep"));
+    if (fused) QWH_TRY(check_hip(ctx, launch_conv_tower_prep(s, ctx->cus, tower, log_mel_dev, frames, ws + off_tower), "front-end prep"));
     if (!ctx->front_table.ptr || ctx->front_table_steps != chunk_steps || ctx->front_table_width != d_model) {
         // addSinusoidalPosition (model.zig:751-763) for the steps of a chunk,
         // in f64 on the host, narrowed to f32 as the reference does; built

@@ -352,7 +352,7 @@ hipError_t launch_conv3x3s2_gelu(hipStream_t s, float *out, const float *in, con
 // enough for its LDS patch: conv_mfma_supported); scratch holds
 // conv_mfma_bytes.
 bool conv_mfma_supported(uint32_t in_ch, uint32_t h, uint32_t w);
-size_t conv_mfma_bytes(uint32_t batch, uint32_t out_ch, uint32_t in_ch, uint32_t h, uint32_t w);
+size_t conv_mfma_bytes(int cus, uint32_t batch, uint32_t out_ch, uint32_t in_ch, uint32_t h, uint32_t w);
 hipError_t launch_conv3x3s2_gelu_mfma(hipStream_t s, int cus, float *out, const float *in, const uint16_t *weights,
                                       const float *bias, uint32_t batch, uint32_t out_ch, uint32_t in_ch, uint32_t h,
                                       uint32_t w, void *scratch);
@@ -366,8 +366,8 @@ struct ConvTower {
     uint32_t bins = 0, chunk_frames = 0, channels = 0, group = 0;
 };
 bool conv_tower_supported(const ConvTower &c);
-size_t conv_tower_bytes(const ConvTower &c);
-hipError_t launch_conv_tower_prep(hipStream_t s, const ConvTower &c, const float *mel, uint32_t frames, void *scratch);
+size_t conv_tower_bytes(int cus, const ConvTower &c);
+hipError_t launch_conv_tower_prep(hipStream_t s, int cus, const ConvTower &c, const float *mel, uint32_t frames, void *scratch);
 hipError_t launch_conv_tower(hipStream_t s, int cus, const ConvTower &c, const float *mel, uint32_t frames, uint32_t first,
                              uint32_t count, float *out, void *scratch);
 hipError_t launch_gather_chunks(hipStream_t s, const float *mel, uint32_t bins, uint32_t frames, uint32_t chunk_frames,

@@ -125,8 +125,9 @@ __global__ __launch_bounds__(256) void conv3x3s2_gelu_kernel(const ConvArgs a) {
 // tests for the border.
 //
 // Workgroup: 256 output channels (four wavefronts of 64) x 64 positions (or 32,
-// where the grid is small: launch_mfma); a wavefront's 64 x 64 tile takes eight products from four LDS words and two
-// weight words a lane. A stage's patch (at most 2 * ceil(63 / ow) + 3 rows) is
+// where the grid is small: launch_mfma, which may also split the stages over
+// workgroups); a wavefront's 64 x 64 tile takes eight products from four LDS
+// words and two weight words a lane. A stage's patch (at most 2 * ceil(63 / ow) + 3 rows) is
 // copied by global-to-LDS loads one stage ahead, and a tap's weights, stored
 // in operand order, are loaded a whole stage before their use. Bound by the
 // matrix cores (about 40 % of their rate, the LDS reads at half of theirs) and
@@ -141,6 +142,7 @@ constexpr int kMfOc = 256;       // output channels per workgroup, 64 per wavefr
 constexpr int kMfPos = 64;       // output positions per workgroup at most (one or two 32-column MFMA tiles)
 constexpr int kMfIc = 16;        // input channels per stage
 constexpr int kMfRounds = 9;     // patch words per thread at most
+constexpr uint32_t kConvMaxSlices = 6;
 
 // A tensor in the halves layout: padded planes of (h + 2) rows x 2 parities x
 // slots words.
@@ -162,6 +164,9 @@ struct ConvMfmaArgs {
     uint8_t *halves;             // the output in the halves layout, or null
     uint32_t out_ch, oc_tiles, stages, h, w, oh, ow, positions;
     uint32_t patch_rows, pos_tiles, units, oc_blocks;
+    uint32_t slices, slice_stages;
+    float *part;                 // slices > 1: [slice][batch][out_ch][positions] sums, for conv_finish_kernel
+    uint32_t batch;
 };
 
 // The two terms of v * s.
@@ -190,21 +195,24 @@ __global__ __launch_bounds__(256, 2) void conv3x3s2_gelu_mfma_kernel(const ConvM
     // Consecutive workgroups run on the eight dies in turn: a position tile's
     // channel blocks stay on one die, next to each other.
     const uint32_t die = blockIdx.x & 7, at = blockIdx.x >> 3;
-    const uint32_t unit = at / a.oc_blocks * 8 + die;
+    const uint32_t inner = a.oc_blocks * a.slices;
+    const uint32_t unit = at / inner * 8 + die;
     if (unit >= a.units) return;
     const uint32_t b = unit / a.pos_tiles, p0 = unit % a.pos_tiles * (32 * NT);
-    const uint32_t oc0 = (at % a.oc_blocks) * kMfOc + wave * 64;
+    const uint32_t slice = at % inner / a.oc_blocks, oc_block = at % a.oc_blocks;
+    const uint32_t first_stage = slice * a.slice_stages, last_stage = min(first_stage + a.slice_stages, a.stages) - 1;
+    const uint32_t oc0 = oc_block * kMfOc + wave * 64;
     const HalvesPlane in_plane = halves_plane(a.h, a.w);
     const uint32_t slots = in_plane.slots;
     const uint32_t patch_plane = a.patch_rows * 2 * slots;  // words of a patch plane
     const uint32_t r_first = p0 / a.ow;
 
-    if (HALVES && p0 == 0) {
+    if (HALVES && p0 == 0 && slice == 0) {
         // The output planes' zero border (this workgroup's channels, once per
         // image): the first and last row, and in the others what is left and
         // right of the columns.
         const HalvesPlane o = halves_plane(a.oh, a.ow);
-        const uint32_t first = (at % a.oc_blocks) * (kMfOc / kMfIc);
+        const uint32_t first = oc_block * (kMfOc / kMfIc);
         const uint32_t count = min((uint32_t)(kMfOc / kMfIc), a.out_ch / kMfIc - first) * 4;
         cu4 *to = reinterpret_cast<cu4 *>(a.halves) + ((size_t)b * (a.out_ch / kMfIc) + first) * 4 * o.words;
         for (uint32_t i = t; i < o.words; i += 256) {
@@ -257,13 +265,13 @@ __global__ __launch_bounds__(256, 2) void conv3x3s2_gelu_mfma_kernel(const ConvM
         __builtin_amdgcn_sched_barrier(0);  // (else it sinks to the stage's end)
     };
     cf32x16 acc[2][NT] = {};
-    copy_patch(0, 0);
+    copy_patch(first_stage, 0);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int tap = 0; tap < 9; ++tap) load_tap(0, tap);
-    for (uint32_t s = 0; s < a.stages; ++s) {
-        const int buf = s & 1;
-        const uint32_t next = min(s + 1, a.stages - 1);
+    for (int tap = 0; tap < 9; ++tap) load_tap(first_stage, tap);
+    int buf = 0;
+    for (uint32_t s = first_stage; s <= last_stage; ++s, buf ^= 1) {
+        const uint32_t next = min(s + 1, last_stage);
         // This stage's patch has landed (the 18 weight words a lane loaded
         // after it may still travel), in every wavefront after the barrier;
         // the other buffer was last read before it.
@@ -298,6 +306,22 @@ __global__ __launch_bounds__(256, 2) void conv3x3s2_gelu_mfma_kernel(const ConvM
     if (oc0 >= a.out_ch) return;
     // Value r of a lane: output channel 8 (r / 4) + 4 half + r % 4 of the
     // tile's 32, position column lane % 32.
+    if (a.part) {
+        float *part = a.part + ((size_t)slice * a.batch + b) * a.out_ch * a.positions;
+#pragma unroll
+        for (int j = 0; j < NT; ++j) {
+            const uint32_t pos = p0 + 32 * j + (lane & 31);
+            if (pos >= a.positions) continue;
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    const uint32_t oc = oc0 + 32 * i + 8 * (r / 4) + 4 * half + r % 4;
+                    if (oc < a.out_ch) part[(size_t)oc * a.positions + pos] = acc[i][j][r];
+                }
+        }
+        return;
+    }
     const float inverse = a.scales[1];
     const float up = HALVES ? a.scales[2] : 0.0f;
     const HalvesPlane o = halves_plane(a.oh, a.ow);
@@ -336,6 +360,55 @@ __global__ __launch_bounds__(256, 2) void conv3x3s2_gelu_mfma_kernel(const ConvM
                         if (oc + k < a.out_ch) a.out[((size_t)b * a.out_ch + oc + k) * a.positions + pos] = y[k];
                 }
             }
+    }
+}
+
+// The slices' sums in slice order, scaled, with bias and GELU: a thread takes
+// eight channels of a position (one word of the halves layout).
+template <bool HALVES>
+__global__ __launch_bounds__(256) void conv_finish_kernel(const ConvMfmaArgs a) {
+    const uint32_t words = (a.out_ch + 7) / 8;
+    const uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= (uint64_t)a.batch * words * a.positions) return;
+    const uint32_t pos = (uint32_t)(i % a.positions);
+    const uint32_t oc = (uint32_t)(i / a.positions % words) * 8, b = (uint32_t)(i / a.positions / words);
+    const size_t plane = (size_t)a.batch * a.out_ch * a.positions;
+    float v[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+        const float *p = a.part + ((size_t)b * a.out_ch + min(oc + k, a.out_ch - 1)) * a.positions + pos;
+        float w[kConvMaxSlices];
+#pragma unroll
+        for (uint32_t s = 0; s < kConvMaxSlices; ++s) w[s] = s < a.slices ? p[s * plane] : 0.0f;
+        v[k] = w[0];
+#pragma unroll
+        for (uint32_t s = 1; s < kConvMaxSlices; ++s)
+            if (s < a.slices) v[k] += w[s];
+    }
+    const float inverse = a.scales[1];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) v[k] = dev::gelu(a.bias[min(oc + k, a.out_ch - 1)] + v[k] * inverse);
+    if constexpr (HALVES) {
+        // (out_ch is a multiple of 16.)
+        const HalvesPlane o = halves_plane(a.oh, a.ow);
+        const uint32_t row = pos / a.ow + 1, col = pos % a.ow + 1;
+        const uint32_t word = (row * 2 + (col & 1)) * o.slots + (col >> 1);
+        const float up = a.scales[2];
+        ch8 hi, lo;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            _Float16 p, l;
+            split_half(v[k], up, p, l);
+            hi[k] = p, lo[k] = l;
+        }
+        ch8 *to = reinterpret_cast<ch8 *>(a.halves) +
+                  (((size_t)b * (a.out_ch / kMfIc) + oc / kMfIc) * 4 + (oc >> 3 & 1)) * o.words + word;
+        to[0] = hi;
+        to[(size_t)2 * o.words] = lo;
+    } else {
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+            if (oc + k < a.out_ch) a.out[((size_t)b * a.out_ch + oc + k) * a.positions + pos] = v[k];
     }
 }
 
@@ -675,13 +748,16 @@ size_t halves_image_bytes(uint32_t channels, uint32_t h, uint32_t w) {
 }
 
 template <int NT, bool HALVES>
-hipError_t launch_mfma_tiles(hipStream_t s, ConvMfmaArgs a, uint32_t batch) {
+hipError_t launch_mfma_tiles(hipStream_t s, ConvMfmaArgs a, uint32_t slices) {
     const HalvesPlane p = halves_plane(a.h, a.w);
     a.patch_rows = std::min(mfma_patch_rows(a.ow, 32 * NT), a.h + 2);
     a.pos_tiles = (a.positions + 32 * NT - 1) / (32 * NT);
-    a.units = batch * a.pos_tiles;
+    a.units = a.batch * a.pos_tiles;
     a.oc_blocks = (a.out_ch + kMfOc - 1) / kMfOc;
-    const uint32_t grid = (a.units + 7) / 8 * 8 * a.oc_blocks;
+    a.slice_stages = (a.stages + slices - 1) / slices;
+    a.slices = (a.stages + a.slice_stages - 1) / a.slice_stages;
+    if (a.slices == 1) a.part = nullptr;
+    const uint32_t grid = (a.units + 7) / 8 * 8 * a.oc_blocks * a.slices;
     const uint32_t rounds = (a.patch_rows * 2 * p.slots * 4 + 255) / 256;
     if (rounds <= 2) conv3x3s2_gelu_mfma_kernel<NT, 2, HALVES><<<grid, 256, 0, s>>>(a);
     else if (rounds <= 4) conv3x3s2_gelu_mfma_kernel<NT, 4, HALVES><<<grid, 256, 0, s>>>(a);
@@ -689,6 +765,10 @@ hipError_t launch_mfma_tiles(hipStream_t s, ConvMfmaArgs a, uint32_t batch) {
     else if (rounds <= 8) conv3x3s2_gelu_mfma_kernel<NT, 8, HALVES><<<grid, 256, 0, s>>>(a);
     else if (rounds <= kMfRounds) conv3x3s2_gelu_mfma_kernel<NT, kMfRounds, HALVES><<<grid, 256, 0, s>>>(a);
     else return hipErrorInvalidValue;
+    if (a.slices > 1) {
+        const uint64_t n = (uint64_t)a.batch * ((a.out_ch + 7) / 8) * a.positions;
+        conv_finish_kernel<HALVES><<<(uint32_t)((n + 255) / 256), 256, 0, s>>>(a);
+    }
     return hipGetLastError();
 }
 
@@ -696,16 +776,29 @@ hipError_t launch_mfma_tiles(hipStream_t s, ConvMfmaArgs a, uint32_t batch) {
 // unevenly filled: a compute unit's share took about 42 us a workgroup of 32
 // positions and 63 of 64 (30 stages; 30 s of audio conv3 89 / 82 us, conv2 253
 // / 252; 4 s conv2 54 / 78, conv3 40 / 66; 11 s conv2 122 / 131).
+//
+// A few chunks leave most compute units idle even so, behind a chain of all
+// the stages: the stages are then split over workgroups, as many as fill the
+// device once, and a second pass adds the slices (us, one launch / split in
+// `cus / workgroups`: conv2 44 / 28 of one chunk and 45 / 33 of two, conv3 36 /
+// 15, 36 / 17, of four 36 / 19 and of eight 36 / 25; a second slice of a
+// device more than half full gained nothing).
 template <bool HALVES>
-hipError_t launch_mfma(hipStream_t s, int cus, const ConvMfmaArgs &a, uint32_t batch) {
-    auto share = [&](uint32_t positions) {
-        const uint64_t groups = (uint64_t)batch * ((a.positions + positions - 1) / positions) *
-                                ((a.out_ch + kMfOc - 1) / kMfOc);
-        return (groups + (uint32_t)cus - 1) / (uint32_t)cus;
+hipError_t launch_mfma(hipStream_t s, int cus, ConvMfmaArgs a, uint32_t batch, float *part) {
+    a.batch = batch;
+    a.part = part;
+    auto groups = [&](uint32_t positions) {
+        return (uint64_t)batch * ((a.positions + positions - 1) / positions) * ((a.out_ch + kMfOc - 1) / kMfOc);
     };
-    return 2 * share(32) <= 3 * share(64) ? launch_mfma_tiles<1, HALVES>(s, a, batch)
-                                          : launch_mfma_tiles<2, HALVES>(s, a, batch);
+    auto share = [&](uint32_t positions) { return (groups(positions) + (uint32_t)cus - 1) / (uint32_t)cus; };
+    if (2 * share(32) > 3 * share(64)) return launch_mfma_tiles<2, HALVES>(s, a, 1);
+    const uint64_t fill = std::min<uint64_t>((uint32_t)cus / groups(32), a.stages / 5);
+    return launch_mfma_tiles<1, HALVES>(s, a, (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(kConvMaxSlices, fill)));
 }
+
+// The slices' sums: a split launch has at most `cus` workgroups of 32
+// positions by kMfOc channels.
+size_t conv_part_bytes(int cus) { return (size_t)cus * 32 * kMfOc * sizeof(float); }
 
 ConvMfmaArgs mfma_args(const void *in, const void *wprep, const float *bias, const float *scales, uint32_t out_ch,
                        uint32_t in_ch, uint32_t h, uint32_t w) {
@@ -741,8 +834,8 @@ uint32_t conv_mfma_group(uint32_t batch, uint32_t in_ch, uint32_t h, uint32_t w)
     return (uint32_t)std::min<size_t>(batch, std::max<size_t>(1, kConvGroupBytes / image));
 }
 
-size_t conv_mfma_bytes(uint32_t batch, uint32_t out_ch, uint32_t in_ch, uint32_t h, uint32_t w) {
-    return wprep_bytes(out_ch, in_ch) + norms_bytes(out_ch) + kMaximaBytes + kScaleBytes +
+size_t conv_mfma_bytes(int cus, uint32_t batch, uint32_t out_ch, uint32_t in_ch, uint32_t h, uint32_t w) {
+    return wprep_bytes(out_ch, in_ch) + norms_bytes(out_ch) + kMaximaBytes + kScaleBytes + conv_part_bytes(cus) +
            conv_mfma_group(batch, in_ch, h, w) * halves_image_bytes(in_ch, h, w);
 }
 
@@ -755,7 +848,8 @@ hipError_t launch_conv3x3s2_gelu_mfma(hipStream_t s, int cus, float *out, const 
     float *norms = reinterpret_cast<float *>(at += wprep_bytes(out_ch, in_ch));
     float *partial = reinterpret_cast<float *>(at += norms_bytes(out_ch));
     float *scales = reinterpret_cast<float *>(at += kMaximaBytes);
-    uint8_t *halves = at + kScaleBytes;
+    float *part = reinterpret_cast<float *>(at += kScaleBytes);
+    uint8_t *halves = at + conv_part_bytes(cus);
     ConvPrepArgs p{};
     p.job[0] = {weights, wprep, norms, out_ch, mfma_oc_pad(out_ch), in_ch};
     p.x = in;
@@ -775,7 +869,7 @@ hipError_t launch_conv3x3s2_gelu_mfma(hipStream_t s, int cus, float *out, const 
         to_halves_kernel<<<dim3((halves_plane(h, w).words + 255) / 256, in_ch / 8, n), 256, 0, s>>>(
             in + (size_t)b * in_ch * h * w, in_ch, h, w, scales, halves);
         a.out = out + (size_t)b * out_ch * a.positions;
-        const hipError_t e = launch_mfma<false>(s, cus, a, n);
+        const hipError_t e = launch_mfma<false>(s, cus, a, n, part);
         if (e != hipSuccess) return e;
     }
     return hipGetLastError();
@@ -785,10 +879,10 @@ hipError_t launch_conv3x3s2_gelu_mfma(hipStream_t s, int cus, float *out, const 
 namespace {
 
 struct TowerPieces {
-    size_t wprep2, wprep3, norms2, norms3, partial, scales, halves1, halves2, total;
+    size_t wprep2, wprep3, norms2, norms3, partial, scales, part, halves1, halves2, total;
 };
 
-TowerPieces tower_pieces(const ConvTower &c) {
+TowerPieces tower_pieces(int cus, const ConvTower &c) {
     const uint32_t h1 = (c.bins - 1) / 2 + 1, w1 = (c.chunk_frames - 1) / 2 + 1;
     const uint32_t h2 = (h1 - 1) / 2 + 1, w2 = (w1 - 1) / 2 + 1;
     TowerPieces p{};
@@ -804,6 +898,7 @@ TowerPieces tower_pieces(const ConvTower &c) {
     p.norms3 = take(norms_bytes(c.channels));
     p.partial = take(kMaximaBytes);
     p.scales = take(kScaleBytes);
+    p.part = take(conv_part_bytes(cus));
     p.halves1 = take(piece(c.group * halves_image_bytes(c.channels, h1, w1)));
     p.halves2 = take(piece(c.group * halves_image_bytes(c.channels, h2, w2)));
     p.total = at;
@@ -818,11 +913,11 @@ bool conv_tower_supported(const ConvTower &c) {
     return conv_mfma_supported(c.channels, h1, w1) && conv_mfma_supported(c.channels, h2, w2);
 }
 
-size_t conv_tower_bytes(const ConvTower &c) { return tower_pieces(c).total; }
+size_t conv_tower_bytes(int cus, const ConvTower &c) { return tower_pieces(cus, c).total; }
 
-hipError_t launch_conv_tower_prep(hipStream_t s, const ConvTower &c, const float *mel, uint32_t frames, void *scratch) {
+hipError_t launch_conv_tower_prep(hipStream_t s, int cus, const ConvTower &c, const float *mel, uint32_t frames, void *scratch) {
     uint8_t *base = static_cast<uint8_t *>(scratch);
-    const TowerPieces at = tower_pieces(c);
+    const TowerPieces at = tower_pieces(cus, c);
     const uint32_t pad = mfma_oc_pad(c.channels);
     ConvPrepArgs p{};
     p.job[0] = {c.weights[1], base + at.wprep2, reinterpret_cast<float *>(base + at.norms2), c.channels, pad, c.channels};
@@ -848,7 +943,7 @@ hipError_t launch_conv_tower_prep(hipStream_t s, const ConvTower &c, const float
 hipError_t launch_conv_tower(hipStream_t s, int cus, const ConvTower &c, const float *mel, uint32_t frames, uint32_t first,
                              uint32_t count, float *out, void *scratch) {
     uint8_t *base = static_cast<uint8_t *>(scratch);
-    const TowerPieces at = tower_pieces(c);
+    const TowerPieces at = tower_pieces(cus, c);
     const float *scales = reinterpret_cast<const float *>(base + at.scales);
     const uint32_t h1 = (c.bins - 1) / 2 + 1, w1 = (c.chunk_frames - 1) / 2 + 1;
     Conv1HalvesArgs k{};
@@ -862,12 +957,12 @@ hipError_t launch_conv_tower(hipStream_t s, int cus, const ConvTower &c, const f
     conv1_halves_kernel<<<dim3((halves_plane(h1, w1).words + 255) / 256, c.channels / kMfIc, count), 256, 0, s>>>(k);
     ConvMfmaArgs a = mfma_args(base + at.halves1, base + at.wprep2, c.bias[1], scales, c.channels, c.channels, h1, w1);
     a.halves = base + at.halves2;
-    const hipError_t e = launch_mfma<true>(s, cus, a, count);
+    const hipError_t e = launch_mfma<true>(s, cus, a, count, reinterpret_cast<float *>(base + at.part));
     if (e != hipSuccess) return e;
     ConvMfmaArgs a3 = mfma_args(base + at.halves2, base + at.wprep3, c.bias[2], scales + 2, c.channels, c.channels, a.oh,
                                 a.ow);
     a3.out = out;
-    return launch_mfma<false>(s, cus, a3, count);
+    return launch_mfma<false>(s, cus, a3, count, reinterpret_cast<float *>(base + at.part));
 }
 
 hipError_t launch_gather_chunks(hipStream_t s, const float *mel, uint32_t bins, uint32_t frames, uint32_t chunk_frames,

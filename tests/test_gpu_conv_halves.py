@@ -20,6 +20,9 @@ pytestmark = pytest.mark.gpu
     (5, 48, 48, 31, 3),      # two-column output: the patch is the whole plane
     (40, 300, 16, 33, 17),   # enough workgroups for the 64-position form
     (1, 16, 16, 64, 93),     # the most patch rounds
+    (1, 250, 160, 9, 13),    # ten stages: two slices
+    (2, 257, 176, 5, 7),     # eleven: a slice of six and one of five
+    (1, 480, 480, 7, 25),    # thirty: six slices
 ])
 def test_conv_tiles(ctx, batch, cout, cin, h, w):
     x = normal(batch * cin * h * w, 91, cin + w)
