@@ -451,14 +451,23 @@ __global__ __launch_bounds__(256) void conv_prep_kernel(const ConvPrepArgs a) {
     } else {
         const uint32_t n = block >= a.job[0].oc_pad ? 1 : 0;
         const ConvWeightsJob &j = a.job[n];
-        const uint32_t oc = block - (n ? a.job[0].oc_pad : 0);
+        // Eight consecutive channels, whose words share 128-byte lines, on one
+        // die (block ids run on the eight dies in turn), so that its L2 joins
+        // their stores.
+        const uint32_t id = block - (n ? a.job[0].oc_pad : 0);
+        const uint32_t oc = (id / 64 * 8 + id % 8) * 8 + id / 8 % 8;
         const uint16_t *row = j.weights + (size_t)min(oc, j.out_ch - 1) * j.in_ch * 9;
         // A channel's weights through LDS, kPrepIc input channels at a time;
         // items (stage, channel half, tap) are eight channels' of a tap.
         for (uint32_t ic = 0; ic < j.in_ch; ic += kPrepIc) {
             const uint32_t n = min((uint32_t)kPrepIc, j.in_ch - ic) * 9;
+            uint16_t r[kPrepIc * 9 / 256];  // (all loads first; past the row, its last value again)
+#pragma unroll
+            for (int k = 0; k < kPrepIc * 9 / 256; ++k) r[k] = row[ic * 9 + min(threadIdx.x + 256u * k, n - 1)];
             __syncthreads();
-            for (uint32_t i = threadIdx.x; i < n; i += 256) rows[i] = row[ic * 9 + i];
+#pragma unroll
+            for (int k = 0; k < kPrepIc * 9 / 256; ++k)
+                if (threadIdx.x + 256u * k < n) rows[threadIdx.x + 256u * k] = r[k];
             __syncthreads();
             for (uint32_t i = threadIdx.x; i < n / 8; i += 256) {
                 const uint32_t tap = i % 9, h = i / 9 % 2, stage = ic / kMfIc + i / 18;
