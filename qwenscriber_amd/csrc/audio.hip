@@ -176,29 +176,40 @@ __global__ __launch_bounds__(64 * kWaves) void audio_attention_kernel(AudioAtten
 #pragma unroll
     for (int i = 0; i < kDimsPerLane; ++i) st.acc[i] = 0.0f;
 
+    // A thread's words of a chunk: rows tid / (HD / 4) + kRowStep i at one
+    // column, so the biases are loaded once; a chunk is loaded into registers
+    // while the one before it is folded in (a layer of 390 steps, 14 heads of
+    // 64: 93.2 -> 91.8 us).
+    constexpr int kRowStep = 64 * kWaves / (HD / 4), kLoads = kKeysPerChunk / kRowStep;
+    const int r0 = threadIdx.x / (HD / 4), c = threadIdx.x % (HD / 4) * 4;
+    float4 kw[kLoads], vw[kLoads];
+    const float4 none = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    const float4 kb = a.k_bias ? *reinterpret_cast<const float4 *>(a.k_bias + column + c) : none;
+    const float4 vb = a.v_bias ? *reinterpret_cast<const float4 *>(a.v_bias + column + c) : none;
+    // Every load is unconditional (rows past the window repeat its last row
+    // and are never read back), so all of them are in flight at once.
+    auto load_chunk = [&](uint32_t k0) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < kLoads; ++i) {
+            const uint32_t row = start + min(k0 + (uint32_t)(r0 + kRowStep * i), length - 1);
+            kw[i] = *reinterpret_cast<const float4 *>(a.k + (size_t)row * a.k_stride + column + c);
+            vw[i] = *reinterpret_cast<const float4 *>(a.v + (size_t)row * a.v_stride + column + c);
+        }
+    };
+    load_chunk(0);
     for (uint32_t k0 = 0; k0 < length; k0 += kKeysPerChunk) {
         const uint32_t count = min((uint32_t)kKeysPerChunk, length - k0);
         __syncthreads();
-        // Every load is unconditional (rows past the window repeat its last
-        // row and are never read back), so all of them are in flight at once.
-#pragma unroll 4
-        for (int idx = threadIdx.x; idx < kKeysPerChunk * (HD / 4); idx += 64 * kWaves) {
-            const int r = idx / (HD / 4), c = (idx % (HD / 4)) * 4;
-            const uint32_t row = start + k0 + min((uint32_t)r, count - 1);
-            float4 kv = *reinterpret_cast<const float4 *>(a.k + (size_t)row * a.k_stride + column + c);
-            float4 vv = *reinterpret_cast<const float4 *>(a.v + (size_t)row * a.v_stride + column + c);
-            if (a.k_bias) {
-                const float4 b = *reinterpret_cast<const float4 *>(a.k_bias + column + c);
-                kv.x += b.x, kv.y += b.y, kv.z += b.z, kv.w += b.w;
-            }
-            if (a.v_bias) {
-                const float4 b = *reinterpret_cast<const float4 *>(a.v_bias + column + c);
-                vv.x += b.x, vv.y += b.y, vv.z += b.z, vv.w += b.w;
-            }
-            lds_k[(r * kRow + c) / 4] = kv;
-            lds_v[(r * kRow + c) / 4] = vv;
+#pragma unroll
+        for (int i = 0; i < kLoads; ++i) {
+            float4 kv = kw[i], vv = vw[i];
+            if (a.k_bias) kv.x += kb.x, kv.y += kb.y, kv.z += kb.z, kv.w += kb.w;
+            if (a.v_bias) vv.x += vb.x, vv.y += vb.y, vv.z += vb.z, vv.w += vb.w;
+            lds_k[((r0 + kRowStep * i) * kRow + c) / 4] = kv;
+            lds_v[((r0 + kRowStep * i) * kRow + c) / 4] = vv;
         }
         __syncthreads();
+        if (k0 + kKeysPerChunk < length) load_chunk(k0 + kKeysPerChunk);
         // This wavefront's share of the chunk's keys: [lo, hi).
         const uint32_t lo = count * wave / kWaves, hi = count * (wave + 1) / kWaves;
         uint32_t j = lo;
