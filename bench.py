@@ -652,7 +652,7 @@ def bench_audio(ctx, qa, steps):
         "workload": "Qwen3-ASR-0.6B audio layer, 390 steps, window 104, q4 weights, f32 activations",
         "frontend_30s_ms": front_ms, "frontend_TFLOPs": front_flops / (front_ms * 1e-3) / 1e12,
         "frontend_workload": "3000 mel frames x 128 bins, 30 chunks, 3 convolutions of 480 channels (f16 weights, "
-                             "f32 FMA), conv_out 896 x 7680 q4, 390 rows",
+                             "matrix cores), conv_out 896 x 7680 q4, 390 rows",
         "layer_us": layer_ms * 1e3, "layer_TFLOPs": (layer_flops + att_flops) / (layer_ms * 1e-3) / 1e12,
         "layer_q5_us": layer_q5_ms * 1e3, "layer_q5_TFLOPs": (layer_flops + att_flops) / (layer_q5_ms * 1e-3) / 1e12,
         "tower_18_layers_ms": 18 * layer_ms,
