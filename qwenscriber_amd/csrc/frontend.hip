@@ -132,7 +132,7 @@ __global__ __launch_bounds__(256) void conv3x3s2_gelu_kernel(const ConvArgs a) {
 // in operand order, are loaded a whole stage before their use. Bound by the
 // matrix cores (about 40 % of their rate, the LDS reads at half of theirs) and
 // by the last, partly empty wave of workgroups; 30 s of audio, 480 channels:
-// conv2 (64 x 50 planes) 706 -> 253 us, conv3 204 -> 82 us.
+// conv2 (64 x 50 planes) 706 -> 248 us, conv3 204 -> 77 us.
 typedef _Float16 ch8 __attribute__((ext_vector_type(8)));
 typedef _Float16 ch4 __attribute__((ext_vector_type(4)));
 typedef float cf32x16 __attribute__((ext_vector_type(16)));
