@@ -4,13 +4,17 @@
 //
 // Each token's row is split once into two f16 terms of x * 2^s (s from the
 // row's largest finite magnitude, so |x * 2^s| < 2^14): hi rounded to f16, lo
-// the exact remainder rounded to f16. A value keeps 22 to 23 significant bits
-// of its own, and nothing below 2^-38 of the row's largest is lost, so the
-// split is at least as close as 23-bit integers per 64-value group (the small
-// batch's digit planes). The codes are small integers, exact in f16, and
-// code * term products are exact in f32; the matrix core adds both terms'
-// products of one 64-column group into one f32 partial, which takes the
-// group's f16 scale in one FMA.
+// the exact remainder rounded to f16. A value is kept to 2^-22 of itself or
+// 2^-39 of what s was taken from, whichever is more. A row with a 64-value
+// group 2^-15 or more below its largest takes s from each group instead (an
+// "uneven" row), so the split is at least as close as 23-bit integers per group
+// (the small batch's digit planes) whatever the row holds: one s for a row with
+// a value 1e8 times the others left them 1e-4 of themselves. The codes are
+// small integers, exact in f16, and code * term products are exact in f32; the
+// matrix core adds both terms' products of one group into one f32 partial,
+// which takes the group's f16 scale in one FMA, in a workgroup with an uneven
+// row times the token's 2^-s (2048 x 6144 q8 and 12288 x 2048 q4 at 402 tokens:
+// 44.9 and 58.1 us, 47.1 and 68.0 with all rows uneven).
 //
 // Operands. One v_mfma_f32_32x32x16_f16 multiplies 32 tokens by 32 weight
 // rows over 16 columns: lane l feeds token (or row) l % 32 and 8 columns, so
@@ -126,7 +130,9 @@ struct RowsArgs {
     const uint16_t *scales;
     const uint8_t *data;
     const uint8_t *halves;   // the split activations
-    const float *inverse;    // per token: 2^-s, times 1 / rms with RMSNorm
+    const float *factor;     // per token: 1, or 1 / rms with RMSNorm
+    const float *scale;      // per token: 2^-s, or 0 of an uneven row
+    const float *uneven;     // [32-token tile][group][token]: 2^-s of an uneven row's groups
     float *out;              // tokens x n, or tokens x n / 2 with pairs
     const float *residual;   // optional, tokens x n (may alias out): out = residual + W x; not with pairs
     float *part;             // non-null: [slice][token][n] partial sums instead of out
@@ -158,6 +164,7 @@ __device__ __forceinline__ void rows_block(const RowsArgs &a, uint32_t row_block
     constexpr int D = 3;
     __shared__ u4 al[D][PIECES];
     __shared__ float inv[TT * kTile];
+    __shared__ float4 mult[W][64 / 4];  // a group's 2^-s by token, a copy for each wavefront
     const int tid = threadIdx.x;
     const int lane = tid & 63, wave = tid >> 6;
     const int col = lane & 31, half = lane >> 5;
@@ -179,7 +186,9 @@ __device__ __forceinline__ void rows_block(const RowsArgs &a, uint32_t row_block
         const uint32_t tile = min(tile0 + q / kGroupPieces, tiles - 1);
         ap[m] = reinterpret_cast<const u4 *>(a.halves) + (size_t)tile * a.groups * kGroupPieces + q % kGroupPieces;
     }
-    if (tid < TT * kTile) inv[tid] = a.inverse[min(tile0 * kTile + tid, a.tokens - 1)];
+    // This lane's token in the multipliers' order.
+    const uint32_t my_token = min(tile0 * kTile + (TT == 2 ? lane : col), a.tokens - 1);
+    const float my_scale = a.scale[my_token], my_factor = a.factor[my_token];
 
     f16x acc[TT];
 #pragma unroll
@@ -210,6 +219,11 @@ __device__ __forceinline__ void rows_block(const RowsArgs &a, uint32_t row_block
     };
     load_weights(g0);
     __builtin_amdgcn_sched_barrier(0);
+    // (Before the copies to LDS: with one in flight the compiler waits for
+    // everything.)
+    const bool uneven = __builtin_amdgcn_ballot_w64(my_scale == 0.0f) != 0;  // the same in every wavefront
+    if (tid < TT * kTile) inv[tid] = uneven ? my_factor : __fmul_rn(my_scale, my_factor);
+    __builtin_amdgcn_sched_barrier(0);
     load_acts(g0, 0);
     load_acts(min(g0 + 1, g1 - 1), 1);
     __builtin_amdgcn_s_waitcnt(kWait<PT>);  // the first weights and words (the steps' counts assume a step before)
@@ -229,6 +243,22 @@ __device__ __forceinline__ void rows_block(const RowsArgs &a, uint32_t row_block
             __builtin_memcpy(&v, cs, 2 * CG);
             v >>= 16 * (gc + CG - a.groups);
             __builtin_memcpy(cs, &v, 2 * CG);
+        }
+    };
+    // p = this buffer's group times the codes w.
+    auto multiply = [&](const uint32_t (&w)[CW], f16x (&p)[TT]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int t = 0; t < TT; ++t) p[t] = f16x{};
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            const h8 b = decode<C>(w, s);
+#pragma unroll
+            for (int t = 0; t < TT; ++t) {
+                const u4 *word = &al[buf][t * kGroupPieces + s * 128 + lane];
+                const h8 hi = __builtin_bit_cast(h8, word[0]), lo = __builtin_bit_cast(h8, word[64]);
+                p[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(hi, b, p[t], 0, 0, 0);
+                p[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(lo, b, p[t], 0, 0, 0);
+            }
         }
     };
     // Group gc + i of the chunk taken at gc; `tail`: of the last, shorter chunk.
@@ -253,19 +283,7 @@ __device__ __forceinline__ void rows_block(const RowsArgs &a, uint32_t row_block
             __builtin_amdgcn_sched_barrier(0);
         }
         f16x p[TT];
-#pragma unroll
-        for (int t = 0; t < TT; ++t) p[t] = f16x{};
-#pragma unroll
-        for (int s = 0; s < 4; ++s) {
-            const h8 b = decode<C>(cw[i], s);
-#pragma unroll
-            for (int t = 0; t < TT; ++t) {
-                const u4 *word = &al[buf][t * kGroupPieces + s * 128 + lane];
-                const h8 hi = __builtin_bit_cast(h8, word[0]), lo = __builtin_bit_cast(h8, word[64]);
-                p[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(hi, b, p[t], 0, 0, 0);
-                p[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(lo, b, p[t], 0, 0, 0);
-            }
-        }
+        multiply(cw[i], p);
         const float sv = dev::f16_bits_to_f32((uint16_t)(cs[i / 2] >> (16 * (i % 2))));
 #pragma unroll
         for (int t = 0; t < TT; ++t)
@@ -273,18 +291,54 @@ __device__ __forceinline__ void rows_block(const RowsArgs &a, uint32_t row_block
             for (int k = 0; k < 16; ++k) acc[t][k] = fmaf(p[t][k], sv, acc[t][k]);
         buf = buf == D - 1 ? 0 : buf + 1;
     };
-    // (Whole chunks apart from the last: an exit inside the chunk would make
-    // the compiler's own waits drain the loads in flight.)
-    uint32_t gc = g0;
-    for (; gc + CG <= g1; gc += CG) {
-        take_chunk(gc);
-        static_for<CG>([&](auto at) __attribute__((always_inline)) { step(at, std::false_type{}, gc); });
-    }
-    if (gc < g1) {
-        take_chunk(gc);
-        static_for<CG>([&](auto at) __attribute__((always_inline)) {
-            if (gc + decltype(at)::value < g1) step(at, std::true_type{}, gc);
-        });
+    if (uneven) {
+        // A group at a time, the next one's codes and multipliers loaded
+        // meanwhile (5 to 17 % slower than the loop below).
+        const float *mp = a.uneven + (size_t)(my_token / kTile) * a.groups * kTile + my_token % kTile;
+        uint16_t next_s = sp[g0];
+        float next_m = mp[(size_t)g0 * kTile];
+        for (uint32_t g = g0; g < g1; ++g) {
+            __builtin_amdgcn_s_waitcnt(kWait<0>);
+            __builtin_amdgcn_s_barrier();
+            load_acts(min(g + 2, g1 - 1), buf == 0 ? 2 : buf - 1);
+            uint32_t w[CW];
+#pragma unroll
+            for (int k = 0; k < CW; ++k) w[k] = rw[0][k];
+            const float sv = dev::f16_bits_to_f32(next_s);
+            reinterpret_cast<float *>(mult[wave])[lane] = my_scale == 0.0f ? next_m : my_scale;
+            const uint32_t gn = min(g + 1, g1 - 1);
+            load_codes<C>(wp + (size_t)gn * code_bytes(C), half, rw[0]);
+            next_s = sp[gn];
+            next_m = mp[(size_t)gn * kTile];
+            f16x p[TT];
+            multiply(w, p);
+            __builtin_amdgcn_wave_barrier();
+#pragma unroll
+            for (int t = 0; t < TT; ++t)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const float4 q = mult[wave][t * 8 + 2 * j + half];
+                    acc[t][4 * j] = fmaf(p[t][4 * j], sv * q.x, acc[t][4 * j]);
+                    acc[t][4 * j + 1] = fmaf(p[t][4 * j + 1], sv * q.y, acc[t][4 * j + 1]);
+                    acc[t][4 * j + 2] = fmaf(p[t][4 * j + 2], sv * q.z, acc[t][4 * j + 2]);
+                    acc[t][4 * j + 3] = fmaf(p[t][4 * j + 3], sv * q.w, acc[t][4 * j + 3]);
+                }
+            buf = buf == D - 1 ? 0 : buf + 1;
+        }
+    } else {
+        // (Whole chunks apart from the last: an exit inside the chunk would make
+        // the compiler's own waits drain the loads in flight.)
+        uint32_t gc = g0;
+        for (; gc + CG <= g1; gc += CG) {
+            take_chunk(gc);
+            static_for<CG>([&](auto at) __attribute__((always_inline)) { step(at, std::false_type{}, gc); });
+        }
+        if (gc < g1) {
+            take_chunk(gc);
+            static_for<CG>([&](auto at) __attribute__((always_inline)) {
+                if (gc + decltype(at)::value < g1) step(at, std::true_type{}, gc);
+            });
+        }
     }
 
     __builtin_amdgcn_s_waitcnt(kWait<0>);  // (the last words, copied past the end, before the LDS is given back)
@@ -380,7 +434,7 @@ struct PrepRowsArgs {
     float *x_out;
     uint32_t bytes;            // pair order: 1 for byte codes, 0 for nibbles
     uint8_t *halves;
-    float *inverse;
+    float *factor, *scale, *uneven;
 };
 
 __device__ __forceinline__ void read8(const float *p, float (&v)[8]) {
@@ -430,17 +484,30 @@ __device__ __forceinline__ void input8(const PrepRowsArgs &a, uint32_t t, uint32
     }
 }
 
-// The largest finite magnitude.
-__device__ __forceinline__ float largest8(const float (&v)[8], float m) {
+// The largest finite magnitude of a group, eight values of it in each of eight
+// neighbouring lanes.
+__device__ __forceinline__ float largest8(const float (&v)[8]) {
+    float m = 0.0f;
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
         const float x = fabsf(v[i]);
         m = x < __builtin_inff() ? fmaxf(m, x) : m;
     }
-    return m;
+    m = fmaxf(m, dev::xor_lane<4>(m));
+    m = fmaxf(m, dev::xor_lane<2>(m));
+    return fmaxf(m, dev::xor_lane<1>(m));
 }
 
-__device__ __forceinline__ void split8(const PrepRowsArgs &a, const float (&v)[8], uint32_t t, uint32_t e, float up) {
+// The spread that a row's groups share one s within: their largest magnitudes'
+// exponents.
+constexpr int kEvenSpread = 15;
+
+// `largest`: of the group; `row`: its row's exponent; `even`: the row's spread
+// is within kEvenSpread.
+__device__ __forceinline__ void split8(const PrepRowsArgs &a, const float (&v)[8], uint32_t t, uint32_t e, float largest,
+                                       int row, bool even) {
+    const int ex = even ? row : dev::chunk_exponent(largest);
+    const float up = __builtin_ldexpf(1.0f, 14 - ex);
     h8 hi, lo;
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
@@ -454,6 +521,8 @@ __device__ __forceinline__ void split8(const PrepRowsArgs &a, const float (&v)[8
     uint8_t *to = a.halves + ((((size_t)(t / kTile) * (a.k >> 6) + g) * 4 + s) * 2 * 64 + h * 32 + t % kTile) * 16;
     *reinterpret_cast<h8 *>(to) = hi;
     *reinterpret_cast<h8 *>(to + 64 * 16) = lo;
+    if (!even && (e & 63) == 0)
+        a.uneven[((size_t)(t / kTile) * (a.k >> 6) + g) * kTile + t % kTile] = __builtin_ldexpf(1.0f, ex - 14);
 }
 
 // Workgroup id to token: eight consecutive tokens, whose words share 128-byte
@@ -467,22 +536,32 @@ __device__ __forceinline__ uint32_t prep_token() {
 
 uint32_t prep_grid(uint32_t tokens) { return (tokens + 8 * kDies - 1) / (8 * kDies) * (8 * kDies); }
 
+struct RowSpread {
+    int exponent;
+    bool even;
+};
+
+// From each thread's largest and least group (groups of zeros are left out);
+// lds: two words a wavefront.
+__device__ __forceinline__ RowSpread row_spread(float most, float least, float2 *lds) {
+    most = dev::wave_max(most);
+    least = -dev::wave_max(-least);
+    if ((threadIdx.x & 63) == 0) lds[threadIdx.x >> 6] = make_float2(most, least);
+    __syncthreads();
+    for (uint32_t w = 0; w < blockDim.x >> 6; ++w) {
+        most = fmaxf(most, lds[w].x);
+        least = fminf(least, lds[w].y);
+    }
+    const int exponent = dev::chunk_exponent(most);
+    return {exponent, exponent - dev::chunk_exponent(least) <= kEvenSpread || !(most > 0.0f)};
+}
+
 template <RowsInput::Form F>
 __global__ __launch_bounds__(kPrepThreads) void prep_rows_kernel(const PrepRowsArgs a) {
     __shared__ float red[4];
+    __shared__ float2 spread[4];
     const uint32_t t = prep_token();
     if (t >= a.tokens) return;
-    const uint32_t waves = blockDim.x >> 6, wave = threadIdx.x >> 6;
-    auto block = [&](float v, auto op) {
-        __syncthreads();
-        if ((threadIdx.x & 63) == 0) red[wave] = v;
-        __syncthreads();
-        v = red[0];
-        for (uint32_t w = 1; w < waves; ++w) v = op(v, red[w]);
-        return v;
-    };
-    const auto add = [](float p, float q) { return p + q; };
-    const auto larger = [](float p, float q) { return fmaxf(p, q); };
     const uint32_t stretch = 8 * blockDim.x;
     float v[kPrepPasses][8];
     float sum = 0.0f, factor = 1.0f;
@@ -504,10 +583,14 @@ __global__ __launch_bounds__(kPrepThreads) void prep_rows_kernel(const PrepRowsA
     }
     if constexpr (F == RowsInput::RmsNorm) {
         // math.zig:120-130; the factor joins the token's output multiplier.
-        sum = block(dev::wave_sum(sum), add);
+        sum = dev::wave_sum(sum);
+        if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = sum;
+        __syncthreads();
+        sum = red[0];
+        for (uint32_t w = 1; w < blockDim.x >> 6; ++w) sum += red[w];
         factor = __fdiv_rn(1.0f, __fsqrt_rn(__fadd_rn(__fdiv_rn(sum, (float)a.k), a.eps)));
     }
-    float amax = 0.0f;
+    float largest[kPrepPasses], most = 0.0f, least = __builtin_inff();
 #pragma unroll
     for (int p = 0; p < kPrepPasses; ++p) {
         const uint32_t e = p * stretch + 8 * threadIdx.x;
@@ -517,43 +600,46 @@ __global__ __launch_bounds__(kPrepThreads) void prep_rows_kernel(const PrepRowsA
 #pragma unroll
             for (int i = 0; i < 8; ++i) v[p][i] = __fmul_rn(v[p][i], w[i]);
         }
-        amax = largest8(v[p], amax);
+        largest[p] = largest8(v[p]);
+        most = fmaxf(most, largest[p]);
+        least = largest[p] > 0.0f ? fminf(least, largest[p]) : least;
     }
-    const int ex = dev::chunk_exponent(block(dev::wave_max(amax), larger));
-    const float up = __builtin_ldexpf(1.0f, 14 - ex);
+    const RowSpread row = row_spread(most, least, spread);
 #pragma unroll
     for (int p = 0; p < kPrepPasses; ++p) {
         const uint32_t e = p * stretch + 8 * threadIdx.x;
-        if (e < a.k) split8(a, v[p], t, e, up);
+        if (e < a.k) split8(a, v[p], t, e, largest[p], row.exponent, row.even);
     }
-    if (threadIdx.x == 0) a.inverse[t] = __fmul_rn(__builtin_ldexpf(1.0f, ex - 14), factor);
+    if (threadIdx.x == 0) a.factor[t] = factor, a.scale[t] = row.even ? __builtin_ldexpf(1.0f, row.exponent - 14) : 0.0f;
 }
 
 // Rows of more than kPrepWidest f32 values: read once for the largest, once
 // to split.
 __global__ __launch_bounds__(kPrepThreads) void prep_rows_wide_kernel(const PrepRowsArgs a) {
-    __shared__ float red[4];
+    __shared__ float2 spread[4];
     const uint32_t t = prep_token();
     if (t >= a.tokens) return;
-    float amax = 0.0f, v[8];
+    float v[8], most = 0.0f, least = __builtin_inff();
     for (uint32_t e = 8 * threadIdx.x; e < a.k; e += 8 * kPrepThreads) {
         input8<RowsInput::F32>(a, t, e, v);
-        amax = largest8(v, amax);
+        const float m = largest8(v);
+        most = fmaxf(most, m);
+        least = m > 0.0f ? fminf(least, m) : least;
     }
-    amax = dev::wave_max(amax);
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = amax;
-    __syncthreads();
-    const int ex = dev::chunk_exponent(fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3])));
-    const float up = __builtin_ldexpf(1.0f, 14 - ex);
+    const RowSpread row = row_spread(most, least, spread);
     for (uint32_t e = 8 * threadIdx.x; e < a.k; e += 8 * kPrepThreads) {
         input8<RowsInput::F32>(a, t, e, v);
-        split8(a, v, t, e, up);
+        split8(a, v, t, e, largest8(v), row.exponent, row.even);
     }
-    if (threadIdx.x == 0) a.inverse[t] = __builtin_ldexpf(1.0f, ex - 14);
+    if (threadIdx.x == 0) a.factor[t] = 1.0f, a.scale[t] = row.even ? __builtin_ldexpf(1.0f, row.exponent - 14) : 0.0f;
 }
 
 size_t halves_bytes(uint32_t tokens, uint32_t cols) {
     return (size_t)((tokens + kTile - 1) / kTile) * kTile * cols * 4;
+}
+
+size_t uneven_bytes(uint32_t tokens, uint32_t cols) {
+    return (size_t)((tokens + kTile - 1) / kTile) * kTile * (cols / 64) * sizeof(float);
 }
 
 constexpr int kWaves = 4;
@@ -628,7 +714,7 @@ bool gemm_rows_preferred(const Matrix &w, uint32_t tokens) {
 }
 
 size_t rows_activation_bytes(uint32_t tokens, uint32_t cols) {
-    return halves_bytes(tokens, cols) + (size_t)tokens * sizeof(float);
+    return halves_bytes(tokens, cols) + uneven_bytes(tokens, cols) + 2 * (size_t)tokens * sizeof(float);
 }
 
 size_t rows_partial_bytes(int cus, uint32_t tokens, const Matrix &w) {
@@ -651,7 +737,9 @@ hipError_t launch_prep_rows(hipStream_t s, const RowsInput &in, int format, uint
     p.x_out = in.sums.x_out;
     p.bytes = format == QWH_FORMAT_Q8 ? 1u : 0u;
     p.halves = static_cast<uint8_t *>(acts);
-    p.inverse = reinterpret_cast<float *>(p.halves + halves_bytes(tokens, cols));
+    p.uneven = reinterpret_cast<float *>(p.halves + halves_bytes(tokens, cols));
+    p.factor = reinterpret_cast<float *>(p.halves + halves_bytes(tokens, cols) + uneven_bytes(tokens, cols));
+    p.scale = p.factor + tokens;
     if (p.slices > kRowsMaxSlices || (p.slices && !p.part)) return hipErrorInvalidValue;
     if (in.form == RowsInput::Pairs && (!p.slices || p.part_n != 2 * cols)) return hipErrorInvalidValue;
     if (in.form == RowsInput::RmsNorm && p.slices && (p.part_n != cols || !p.x_out)) return hipErrorInvalidValue;
@@ -682,7 +770,9 @@ hipError_t launch_gemm_rows(hipStream_t s, int cus, const void *acts, const Matr
     a.scales = reinterpret_cast<const uint16_t *>(w.scales);
     a.data = w.data;
     a.halves = static_cast<const uint8_t *>(acts);
-    a.inverse = reinterpret_cast<const float *>(a.halves + halves_bytes(tokens, w.cols));
+    a.uneven = reinterpret_cast<const float *>(a.halves + halves_bytes(tokens, w.cols));
+    a.factor = reinterpret_cast<const float *>(a.halves + halves_bytes(tokens, w.cols) + uneven_bytes(tokens, w.cols));
+    a.scale = a.factor + tokens;
     a.out = out.out;
     a.residual = out.residual;
     a.pairs = out.pairs ? 1u : 0u;

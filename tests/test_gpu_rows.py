@@ -6,6 +6,7 @@ import numpy as np
 import pytest
 
 import qwenscriber_amd as qa
+from oracle import oracle as o
 from util import normal, quantized_matrix
 
 pytestmark = pytest.mark.gpu
@@ -39,6 +40,15 @@ def dequantized(fmt, rows, cols, scales, data):
     return ((u - BIAS[fmt]) * s).reshape(rows, cols)
 
 
+def error_bound(x, w):
+    """Of x times w^T: the values' and the sums' rounding, as the caller says."""
+    tokens, cols = x.shape
+    mass = np.abs(x).astype(np.float64) @ np.abs(w).T
+    largest = np.abs(x).reshape(tokens, -1, 64).max(axis=2).astype(np.float64)
+    floor = largest @ np.abs(w).reshape(w.shape[0], -1, 64).sum(axis=2).T
+    return (cols // 64 + 24) * 2.0 ** -23 * mass + 2.0 ** -39 * floor + 1e-37
+
+
 @pytest.mark.parametrize("fmt", [qa.FORMAT_Q4, qa.FORMAT_Q5, qa.FORMAT_Q8])
 @pytest.mark.parametrize("rows,cols,tokens", [
     (48829, 256, 128),   # the least K and tokens; ragged last row tile
@@ -62,13 +72,10 @@ def test_linear_many_tokens(ctx, fmt, rows, cols, tokens):
     got = run_linear(ctx, fmt, rows, cols, scales, data, x).astype(np.float64)
     w = dequantized(fmt, rows, cols, scales, data)
     want = x.astype(np.float64) @ w.T
-    # Each product carries 2^-22 of its value (two f16 terms) or 2^-36 of the
-    # row's largest (below the f16 range); a sum is rounded at most 9 times
+    # Each product carries 2^-22 of its value (two f16 terms) or 2^-39 of its
+    # group's largest (below the f16 range); a sum is rounded at most 9 times
     # within a group, once per group and slice, and twice at the end.
-    eps = 2.0 ** -23
-    mass = np.abs(x).astype(np.float64) @ np.abs(w).T
-    floor = np.abs(x).max(axis=1, keepdims=True).astype(np.float64) * np.abs(w).sum(axis=1)[None, :]
-    bound = (cols // 64 + 24) * eps * mass + 2.0 ** -36 * floor + 1e-37
+    bound = error_bound(x, w)
     worst = np.abs(got - want) / bound
     assert worst.max() <= 1.0, (worst.max(), np.unravel_index(worst.argmax(), worst.shape))
 
@@ -86,3 +93,21 @@ def test_linear_many_tokens_non_finite(ctx, fmt):
     others = [t for t in range(tokens) if t not in (7, 21)]
     assert np.array_equal(got[others], clean[others])
     assert not np.isfinite(got[7]).any() and np.isnan(got[21]).all()
+
+
+@pytest.mark.parametrize("fmt", [qa.FORMAT_Q4, qa.FORMAT_Q5, qa.FORMAT_Q8])
+@pytest.mark.parametrize("outlier", [1e6, 1e12, 1e25])
+def test_linear_many_tokens_outlier_group(ctx, fmt, outlier):
+    # A group far above its row, under weights that are zero there, takes
+    # nothing from the other groups' precision.
+    rows, cols, tokens = 6400, 2048, 160
+    values = normal(rows * cols, 10, 1, 0.02).reshape(rows, cols)
+    values[:, 640:704] = 0.0
+    scales, data = o.quantize_rows(fmt, values)
+    x = normal(tokens * cols, 11, 2).reshape(tokens, cols)
+    x[:, 650] = np.float32(outlier)
+    got = run_linear(ctx, fmt, rows, cols, scales, data, x).astype(np.float64)
+    w = dequantized(fmt, rows, cols, scales, data)
+    assert not w[:, 640:704].any()
+    worst = np.abs(got - x.astype(np.float64) @ w.T) / error_bound(x, w)
+    assert worst.max() <= 1.0, worst.max()
