@@ -1167,7 +1167,8 @@ int32_t qwh_audio_frontend(qwh_ctx *ctx, const qwh_audio_frontend_weights *w, co
     ConvTower tower;
     tower.weights[0] = w->conv1_weight, tower.weights[1] = w->conv2_weight, tower.weights[2] = w->conv3_weight;
     tower.bias[0] = w->conv1_bias, tower.bias[1] = w->conv2_bias, tower.bias[2] = w->conv3_bias;
-    tower.bins = mel_bins, tower.chunk_frames = chunk_frames, tower.channels = downsample, tower.group = group;
+    tower.bins = mel_bins, tower.chunk_frames = chunk_frames, tower.channels = downsample;
+    tower.chunks = chunks, tower.group = group;
     const bool fused = conv_tower_supported(tower);
     const size_t off1 = fused ? 0 : align(group * mel_plane), off2 = off1 + (fused ? 0 : align(group * p1));
     const size_t off3 = off2 + (fused ? 0 : align(group * p2));

@@ -357,13 +357,13 @@ hipError_t launch_conv3x3s2_gelu_mfma(hipStream_t s, int cus, float *out, const 
                                       const float *bias, uint32_t batch, uint32_t out_ch, uint32_t in_ch, uint32_t h,
                                       uint32_t w, void *scratch);
 // The tower's three convolutions over chunks of chunk_frames frames of a
-// log-mel, up to `group` chunks at a time, where conv2 and conv3 have that
+// log-mel, `chunks` of them, up to `group` at a time, where conv2 and conv3 have that
 // form: the intermediate planes stay in its layout. launch_conv_tower_prep
 // once per call, then each run of chunks to out [count][channels][h3][w3].
 struct ConvTower {
     const uint16_t *weights[3] = {};
     const float *bias[3] = {};
-    uint32_t bins = 0, chunk_frames = 0, channels = 0, group = 0;
+    uint32_t bins = 0, chunk_frames = 0, channels = 0, chunks = 0, group = 0;
 };
 bool conv_tower_supported(const ConvTower &c);
 size_t conv_tower_bytes(int cus, const ConvTower &c);

@@ -109,12 +109,14 @@ __global__ __launch_bounds__(256) void conv3x3s2_gelu_kernel(const ConvArgs a) {
 // output channels, columns are output positions (row-major over the output
 // plane), and the reduction runs over (tap, input channel) in stages of 16
 // input channels, one 16-deep MFMA step per tap. A weight is f16 as it is. An
-// activation is two f16 terms of x * s: hi its f16 rounding, lo the exact
-// remainder rounded to f16, with s a power of two for the whole tensor from a
+// activation is two f16 terms of x * s: hi its f16 rounding, lo 2^11 times the
+// exact remainder rounded to f16, with s a power of two for the image from a
 // bound on its largest magnitude, |x * s| < 2^15. So a value keeps 22
-// significant bits, and nothing above 2^-40 of the bound is lost; the
-// products are exact and summed in f32 by the matrix core. (Two bf16 terms of
-// both operands, without a scale, took four products a tap and kept 2^-17.)
+// significant bits down to 2^-29 of the bound, and nothing above 2^-51 of it is
+// lost, whatever the other images hold; the products are exact and summed in
+// f32 by the matrix core, each term's in accumulators of its own. (Two bf16
+// terms of both operands, without a scale, took four products a tap and kept
+// 2^-17.)
 //
 // The terms are stored once by whoever makes the activations (the "halves"
 // layout): [image][stage][plane][row][parity][slot] 16-byte words of 8
@@ -159,21 +161,22 @@ struct ConvMfmaArgs {
     const uint8_t *in;           // halves
     const uint8_t *wprep;        // [stage][tap][oc / 32][lane][8] f16
     const float *bias;
-    const float *scales;         // input: 2^-e; halves output: also its 2^e
+    const float *scales;         // per image, scale_stride apart: input [1]: 2^-e; halves output [2]: its 2^e
     float *out;                  // [batch][out_ch][oh * ow] f32, or null
     uint8_t *halves;             // the output in the halves layout, or null
     uint32_t out_ch, oc_tiles, stages, h, w, oh, ow, positions;
     uint32_t patch_rows, pos_tiles, units, oc_blocks;
-    uint32_t slices, slice_stages;
+    uint32_t slices, slice_stages, scale_stride;
     float *part;                 // slices > 1: [slice][batch][out_ch][positions] sums, for conv_finish_kernel
     uint32_t batch;
 };
 
-// The two terms of v * s.
+// The two terms of v * s, the second times 2^11.
+constexpr float kLoUp = 2048.0f, kLoDown = 1.0f / 2048.0f;
 __device__ __forceinline__ void split_half(float v, float s, _Float16 &hi, _Float16 &lo) {
     const float x = v * s;
     hi = (_Float16)x;
-    const float rest = x - (float)hi;
+    const float rest = (x - (float)hi) * kLoUp;
     lo = fabsf(rest) < __builtin_inff() ? (_Float16)rest : (_Float16)0.0f;  // (inf and NaN are hi's)
 }
 
@@ -185,12 +188,13 @@ constexpr int kConvWait = (N & 15) | (7 << 4) | ((N >> 4) << 14);
 template <int N>
 constexpr int kConvLoads = kConvWait<N> | (15 << 8);
 
-// NT: 32-position tiles; R: rounds of 256 patch words.
+// NT: 32-position tiles; R: rounds of 256 patch words. (Three workgroups a CU
+// where their LDS allows it: one register more would leave two.)
 template <int NT, int R, bool HALVES>
-__global__ __launch_bounds__(256, 2) void conv3x3s2_gelu_mfma_kernel(const ConvMfmaArgs a) {
+__global__ __launch_bounds__(256, NT == 1 && R <= 6 ? 3 : 2) void conv3x3s2_gelu_mfma_kernel(const ConvMfmaArgs a) {
     __shared__ cu4 patch[2][R * 256];
     const int t = threadIdx.x;
-    const int lane = t & 63, wave = t >> 6;
+    const int lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
     const int half = lane >> 5;
     // Consecutive workgroups run on the eight dies in turn: a position tile's
     // channel blocks stay on one die, next to each other.
@@ -264,7 +268,7 @@ __global__ __launch_bounds__(256, 2) void conv3x3s2_gelu_mfma_kernel(const ConvM
         wa[tap][1] = __builtin_bit_cast(ch8, src[64]);
         __builtin_amdgcn_sched_barrier(0);  // (else it sinks to the stage's end)
     };
-    cf32x16 acc[2][NT] = {};
+    cf32x16 acc[2][NT] = {}, acc_lo[2][NT] = {};
     copy_patch(first_stage, 0);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -296,38 +300,49 @@ __global__ __launch_bounds__(256, 2) void conv3x3s2_gelu_mfma_kernel(const ConvM
 #pragma unroll
                 for (int i = 0; i < 2; ++i)
 #pragma unroll
-                    for (int j = 0; j < NT; ++j)
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(wa[tap][i], x[j], acc[i][j], 0, 0, 0);
+                    for (int j = 0; j < NT; ++j) {
+                        cf32x16 &to = term ? acc_lo[i][j] : acc[i][j];
+                        to = __builtin_amdgcn_mfma_f32_32x32x16_f16(wa[tap][i], x[j], to, 0, 0, 0);
+                    }
             }
             load_tap(next, tap);
         }
     }
     __builtin_amdgcn_s_waitcnt(kConvWait<0>);  // (the last copy, unused, before the LDS is given back)
     if (oc0 >= a.out_ch) return;
+    // (Computed again: no register of the loop's, at its limit, holds them.)
+    const int out_lane = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)), out_half = out_lane >> 5;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[i][j][r] = fmaf(acc_lo[i][j][r], kLoDown, acc[i][j][r]);
     // Value r of a lane: output channel 8 (r / 4) + 4 half + r % 4 of the
     // tile's 32, position column lane % 32.
     if (a.part) {
         float *part = a.part + ((size_t)slice * a.batch + b) * a.out_ch * a.positions;
 #pragma unroll
         for (int j = 0; j < NT; ++j) {
-            const uint32_t pos = p0 + 32 * j + (lane & 31);
+            const uint32_t pos = p0 + 32 * j + (out_lane & 31);
             if (pos >= a.positions) continue;
 #pragma unroll
             for (int i = 0; i < 2; ++i)
 #pragma unroll
                 for (int r = 0; r < 16; ++r) {
-                    const uint32_t oc = oc0 + 32 * i + 8 * (r / 4) + 4 * half + r % 4;
+                    const uint32_t oc = oc0 + 32 * i + 8 * (r / 4) + 4 * out_half + r % 4;
                     if (oc < a.out_ch) part[(size_t)oc * a.positions + pos] = acc[i][j][r];
                 }
         }
         return;
     }
-    const float inverse = a.scales[1];
-    const float up = HALVES ? a.scales[2] : 0.0f;
+    const float *scales = a.scales + (size_t)b * a.scale_stride;
+    const float inverse = scales[1];
+    const float up = HALVES ? scales[2] : 0.0f;
     const HalvesPlane o = halves_plane(a.oh, a.ow);
 #pragma unroll
     for (int j = 0; j < NT; ++j) {
-        const uint32_t pos = p0 + 32 * j + (lane & 31);
+        const uint32_t pos = p0 + 32 * j + (out_lane & 31);
         if (pos >= a.positions) continue;
         const uint32_t row = pos / a.ow + 1, col = pos % a.ow + 1;
         const uint32_t word = (row * 2 + (col & 1)) * o.slots + (col >> 1);
@@ -335,7 +350,7 @@ __global__ __launch_bounds__(256, 2) void conv3x3s2_gelu_mfma_kernel(const ConvM
         for (int i = 0; i < 2; ++i)
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
-                const uint32_t oc = oc0 + 32 * i + 8 * q + 4 * half;
+                const uint32_t oc = oc0 + 32 * i + 8 * q + 4 * out_half;
                 if (oc >= a.out_ch) continue;
                 float y[4];
 #pragma unroll
@@ -351,7 +366,7 @@ __global__ __launch_bounds__(256, 2) void conv3x3s2_gelu_mfma_kernel(const ConvM
                     }
                     // (Channels oc .. oc + 3 are half of a word of eight.)
                     uint8_t *to = a.halves + ((((size_t)b * (a.out_ch / kMfIc) + oc / kMfIc) * 4 + (q & 1)) * o.words +
-                                              word) * 16 + 8 * half;
+                                              word) * 16 + 8 * out_half;
                     *reinterpret_cast<ch4 *>(to) = hi;
                     *reinterpret_cast<ch4 *>(to + (size_t)2 * o.words * 16) = lo;
                 } else {
@@ -385,7 +400,8 @@ __global__ __launch_bounds__(256) void conv_finish_kernel(const ConvMfmaArgs a) 
         for (uint32_t s = 1; s < kConvMaxSlices; ++s)
             if (s < a.slices) v[k] += w[s];
     }
-    const float inverse = a.scales[1];
+    const float *scales = a.scales + (size_t)b * a.scale_stride;
+    const float inverse = scales[1];
 #pragma unroll
     for (int k = 0; k < 8; ++k) v[k] = dev::gelu(a.bias[min(oc + k, a.out_ch - 1)] + v[k] * inverse);
     if constexpr (HALVES) {
@@ -393,7 +409,7 @@ __global__ __launch_bounds__(256) void conv_finish_kernel(const ConvMfmaArgs a) 
         const HalvesPlane o = halves_plane(a.oh, a.ow);
         const uint32_t row = pos / a.ow + 1, col = pos % a.ow + 1;
         const uint32_t word = (row * 2 + (col & 1)) * o.slots + (col >> 1);
-        const float up = a.scales[2];
+        const float up = scales[2];
         ch8 hi, lo;
 #pragma unroll
         for (int k = 0; k < 8; ++k) {
@@ -415,7 +431,8 @@ __global__ __launch_bounds__(256) void conv_finish_kernel(const ConvMfmaArgs a) 
 // What a call prepares: each convolution's weights in operand order with the
 // sum of magnitudes per output channel (a workgroup per channel; channels
 // past out_ch are zero), and the partial maxima of |x| over finite values of
-// an input (the workgroups after them).
+// each image of an input (the workgroups after them, `partials` to an image, four
+// rows to a wavefront).
 struct ConvWeightsJob {
     const uint16_t *weights;     // [out_ch][in_ch][9] f16 bits
     uint8_t *wprep;
@@ -425,9 +442,12 @@ struct ConvWeightsJob {
 
 struct ConvPrepArgs {
     ConvWeightsJob job[2];
+    // Row r of image b: x + b * image_stride + r * row_stride, row_values
+    // values, of which those below row_limit - b * image_stride exist.
     const float *x;
-    uint64_t count;
-    float *partial;
+    uint64_t image_stride, row_stride, row_limit, row_values;
+    uint32_t rows;
+    float *partial;              // [image][partials]
     uint32_t partials;
 };
 
@@ -442,9 +462,20 @@ __global__ __launch_bounds__(256) void conv_prep_kernel(const ConvPrepArgs a) {
     const bool maxima = block >= a.job[0].oc_pad + a.job[1].oc_pad;
     if (maxima) {
         block -= a.job[0].oc_pad + a.job[1].oc_pad;
-        for (uint64_t i = (uint64_t)block * 256 + threadIdx.x; i < a.count; i += (uint64_t)a.partials * 256) {
-            const float m = fabsf(a.x[i]);
-            v = m < __builtin_inff() ? fmaxf(v, m) : v;
+        const uint64_t first = block / a.partials * a.image_stride;
+        const uint64_t n = min(a.row_values, a.row_limit - first);
+        // (Four rows' loads at a time; past the last row, that row again.)
+        for (uint32_t r = (block % a.partials * 4 + (threadIdx.x >> 6)) * 4; r < a.rows; r += a.partials * 16) {
+            const float *row[4];
+#pragma unroll
+            for (uint32_t k = 0; k < 4; ++k) row[k] = a.x + first + min(r + k, a.rows - 1) * a.row_stride;
+            for (uint64_t i = threadIdx.x & 63; i < n; i += 64) {
+                float m[4];
+#pragma unroll
+                for (int k = 0; k < 4; ++k) m[k] = fabsf(row[k][i]);
+#pragma unroll
+                for (int k = 0; k < 4; ++k) v = m[k] < __builtin_inff() ? fmaxf(v, m[k]) : v;
+            }
         }
         v = dev::wave_max(v);
         to = a.partial + block;
@@ -491,19 +522,19 @@ __global__ __launch_bounds__(256) void conv_prep_kernel(const ConvPrepArgs a) {
         *to = maxima ? fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3])) : (red[0] + red[1]) + (red[2] + red[3]);
 }
 
-// The tensors' scales {2^e, 2^-e} from bounds on their magnitudes: the first
-// from the partial maxima of the input -- that input itself, or (conv1) the
-// result of a one-channel convolution of it -- and the next from the first's
-// bound through a convolution's weight sums: |gelu(y)| <= |y| <= |bias| + sum
-// |w| * bound. (A bound a thousand times the largest value still keeps it to
-// 2^-30.)
+// An image's scales {2^e, 2^-e} from bounds on its magnitudes, one workgroup
+// an image: the first from the partial maxima of the input -- that input
+// itself, or (conv1) the result of a one-channel convolution of it -- and the
+// next from the first's bound through a convolution's weight sums: |gelu(y)|
+// <= |y| <= |bias| + sum |w| * bound. (A bound a thousand times the largest
+// value still keeps it to 2^-41.)
 struct ConvScaleArgs {
     const float *partial;
     uint32_t partials;
     const uint16_t *conv1;       // [channels][9] f16 bits, or null
     const float *bias1, *norms2, *bias2;  // norms2 null: the first scale only
     uint32_t channels;
-    float *scales;               // {s, 1 / s} of the first, then of the next
+    float *scales;               // per image, {s, 1 / s} of the first, then (norms2) of the next
 };
 
 __device__ __forceinline__ float block_max_256(float v, float *red) {
@@ -517,7 +548,8 @@ __device__ __forceinline__ float block_max_256(float v, float *red) {
 __global__ __launch_bounds__(256) void conv_scale_kernel(const ConvScaleArgs a) {
     __shared__ float red[4];
     float v = 0.0f;
-    for (uint32_t i = threadIdx.x; i < a.partials; i += 256) v = fmaxf(v, a.partial[i]);
+    for (uint32_t i = threadIdx.x; i < a.partials; i += 256) v = fmaxf(v, a.partial[(size_t)blockIdx.x * a.partials + i]);
+    float *scales = a.scales + (size_t)blockIdx.x * (a.norms2 ? 4 : 2);
     float bound = block_max_256(v, red);
     auto emit = [&](float m, float *to) {
         // 2^e > m, with room for the bound's own rounding.
@@ -533,17 +565,17 @@ __global__ __launch_bounds__(256) void conv_scale_kernel(const ConvScaleArgs a) 
         }
         bound = block_max_256(v, red);
     }
-    emit(bound, a.scales);
+    emit(bound, scales);
     if (!a.norms2) return;
     v = 0.0f;
     for (uint32_t c = threadIdx.x; c < a.channels; c += 256) v = fmaxf(v, fabsf(a.bias2[c]) + a.norms2[c] * bound);
-    emit(block_max_256(v, red), a.scales + 2);
+    emit(block_max_256(v, red), scales + 2);
 }
 
 // f32 [image][channel][h][w] to the halves layout, border included: a thread
 // per word pair (both terms), channels in groups of eight.
 __global__ __launch_bounds__(256) void to_halves_kernel(const float *in, uint32_t channels, uint32_t h, uint32_t w,
-                                                        const float *scales, uint8_t *out) {
+                                                        const float *scales, uint8_t *out) {  // (scales: an image's two)
     const HalvesPlane p = halves_plane(h, w);
     const uint32_t i = blockIdx.x * 256 + threadIdx.x;
     if (i >= p.words) return;
@@ -551,7 +583,7 @@ __global__ __launch_bounds__(256) void to_halves_kernel(const float *in, uint32_
     const uint32_t row = i / (2 * p.slots), rest = i % (2 * p.slots);
     const uint32_t col = 2 * (rest % p.slots) + rest / p.slots;
     const bool inside = row >= 1 && row <= h && col >= 1 && col <= w;
-    const float up = scales[0];
+    const float up = scales[2 * (size_t)b];
     const float *src = in + (((size_t)b * channels + c0) * h + (inside ? row - 1 : 0)) * w + (inside ? col - 1 : 0);
     ch8 hi, lo;
 #pragma unroll
@@ -574,7 +606,7 @@ __global__ __launch_bounds__(256) void to_halves_kernel(const float *in, uint32_
 struct Conv1HalvesArgs {
     const float *mel;
     const uint16_t *weights;
-    const float *bias, *scales;
+    const float *bias, *scales;  // (four scales an image)
     uint8_t *out;
     uint32_t bins, frames, chunk_frames, first, channels, oh, ow;
 };
@@ -607,7 +639,7 @@ __global__ __launch_bounds__(256) void conv1_halves_kernel(const Conv1HalvesArgs
         ok[tap] = r >= 0 && r < (int)a.bins && c >= 0 && c < (int)a.chunk_frames;
         x[tap] = ok[tap] && frame0 + c < a.frames ? a.mel[(size_t)r * a.frames + frame0 + c] : 0.0f;
     }
-    const float up = a.scales[0];
+    const float up = a.scales[4 * (size_t)b];
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
         ch8 hi, lo;
@@ -742,15 +774,17 @@ uint32_t mfma_patch_rows(uint32_t ow, uint32_t positions = kMfPos) { return 2 * 
 
 uint32_t mfma_oc_pad(uint32_t out_ch) { return (out_ch + 63) / 64 * 64; }
 
-constexpr uint32_t kMaximaBlocks = 256;
+// Workgroups that look for an image's largest magnitude: four rows a wavefront
+// and more.
+uint32_t maxima_blocks(uint32_t rows) { return std::min(16u, (rows + 15) / 16); }
 
 // Workspace pieces of a prepared convolution: operand-order weights, channel
 // sums, partial maxima and scales, 256-byte aligned.
 size_t piece(size_t bytes) { return (bytes + 255) & ~(size_t)255; }
 size_t wprep_bytes(uint32_t out_ch, uint32_t in_ch) { return piece((size_t)mfma_oc_pad(out_ch) * in_ch * 9 * 2); }
 size_t norms_bytes(uint32_t out_ch) { return piece((size_t)mfma_oc_pad(out_ch) * sizeof(float)); }
-constexpr size_t kMaximaBytes = kMaximaBlocks * sizeof(float);
-constexpr size_t kScaleBytes = 256;
+size_t maxima_bytes(uint32_t images, uint32_t rows) { return piece((size_t)images * maxima_blocks(rows) * sizeof(float)); }
+size_t scale_bytes(uint32_t images) { return piece((size_t)images * 4 * sizeof(float)); }
 
 size_t halves_image_bytes(uint32_t channels, uint32_t h, uint32_t w) {
     return (size_t)channels / kMfIc * 4 * halves_plane(h, w).words * 16;
@@ -809,13 +843,14 @@ hipError_t launch_mfma(hipStream_t s, int cus, ConvMfmaArgs a, uint32_t batch, f
 // positions by kMfOc channels.
 size_t conv_part_bytes(int cus) { return (size_t)cus * 32 * kMfOc * sizeof(float); }
 
-ConvMfmaArgs mfma_args(const void *in, const void *wprep, const float *bias, const float *scales, uint32_t out_ch,
-                       uint32_t in_ch, uint32_t h, uint32_t w) {
+ConvMfmaArgs mfma_args(const void *in, const void *wprep, const float *bias, const float *scales, uint32_t scale_stride,
+                       uint32_t out_ch, uint32_t in_ch, uint32_t h, uint32_t w) {
     ConvMfmaArgs a{};
     a.in = static_cast<const uint8_t *>(in);
     a.wprep = static_cast<const uint8_t *>(wprep);
     a.bias = bias;
     a.scales = scales;
+    a.scale_stride = scale_stride;
     a.out_ch = out_ch;
     a.oc_tiles = mfma_oc_pad(out_ch) / 32;
     a.stages = in_ch / kMfIc;
@@ -844,7 +879,8 @@ uint32_t conv_mfma_group(uint32_t batch, uint32_t in_ch, uint32_t h, uint32_t w)
 }
 
 size_t conv_mfma_bytes(int cus, uint32_t batch, uint32_t out_ch, uint32_t in_ch, uint32_t h, uint32_t w) {
-    return wprep_bytes(out_ch, in_ch) + norms_bytes(out_ch) + kMaximaBytes + kScaleBytes + conv_part_bytes(cus) +
+    return wprep_bytes(out_ch, in_ch) + norms_bytes(out_ch) + maxima_bytes(batch, in_ch) + scale_bytes(batch) +
+           conv_part_bytes(cus) +
            conv_mfma_group(batch, in_ch, h, w) * halves_image_bytes(in_ch, h, w);
 }
 
@@ -856,27 +892,31 @@ hipError_t launch_conv3x3s2_gelu_mfma(hipStream_t s, int cus, float *out, const 
     uint8_t *wprep = at;
     float *norms = reinterpret_cast<float *>(at += wprep_bytes(out_ch, in_ch));
     float *partial = reinterpret_cast<float *>(at += norms_bytes(out_ch));
-    float *scales = reinterpret_cast<float *>(at += kMaximaBytes);
-    float *part = reinterpret_cast<float *>(at += kScaleBytes);
+    float *scales = reinterpret_cast<float *>(at += maxima_bytes(batch, in_ch));
+    float *part = reinterpret_cast<float *>(at += scale_bytes(batch));
     uint8_t *halves = at + conv_part_bytes(cus);
     ConvPrepArgs p{};
     p.job[0] = {weights, wprep, norms, out_ch, mfma_oc_pad(out_ch), in_ch};
     p.x = in;
-    p.count = (uint64_t)batch * in_ch * h * w;
+    p.rows = in_ch;
+    p.row_values = p.row_stride = (uint64_t)h * w;
+    p.image_stride = in_ch * p.row_stride;
+    p.row_limit = batch * p.image_stride;
     p.partial = partial;
-    p.partials = (uint32_t)std::min<uint64_t>(kMaximaBlocks, (p.count + 255) / 256);
-    conv_prep_kernel<<<p.job[0].oc_pad + p.partials, 256, 0, s>>>(p);
+    p.partials = maxima_blocks(in_ch);
+    conv_prep_kernel<<<p.job[0].oc_pad + batch * p.partials, 256, 0, s>>>(p);
     ConvScaleArgs c{};
     c.partial = partial;
     c.partials = p.partials;
     c.scales = scales;
-    conv_scale_kernel<<<1, 256, 0, s>>>(c);
-    ConvMfmaArgs a = mfma_args(halves, wprep, bias, scales, out_ch, in_ch, h, w);
+    conv_scale_kernel<<<batch, 256, 0, s>>>(c);
+    ConvMfmaArgs a = mfma_args(halves, wprep, bias, scales, 2, out_ch, in_ch, h, w);
     const uint32_t group = conv_mfma_group(batch, in_ch, h, w);
     for (uint32_t b = 0; b < batch; b += group) {
         const uint32_t n = std::min(group, batch - b);
         to_halves_kernel<<<dim3((halves_plane(h, w).words + 255) / 256, in_ch / 8, n), 256, 0, s>>>(
-            in + (size_t)b * in_ch * h * w, in_ch, h, w, scales, halves);
+            in + (size_t)b * in_ch * h * w, in_ch, h, w, scales + 2 * (size_t)b, halves);
+        a.scales = scales + 2 * (size_t)b;
         a.out = out + (size_t)b * out_ch * a.positions;
         const hipError_t e = launch_mfma<false>(s, cus, a, n, part);
         if (e != hipSuccess) return e;
@@ -905,8 +945,8 @@ TowerPieces tower_pieces(int cus, const ConvTower &c) {
     p.wprep3 = take(wprep_bytes(c.channels, c.channels));
     p.norms2 = take(norms_bytes(c.channels));
     p.norms3 = take(norms_bytes(c.channels));
-    p.partial = take(kMaximaBytes);
-    p.scales = take(kScaleBytes);
+    p.partial = take(maxima_bytes(c.chunks, c.bins));
+    p.scales = take(scale_bytes(c.chunks));
     p.part = take(conv_part_bytes(cus));
     p.halves1 = take(piece(c.group * halves_image_bytes(c.channels, h1, w1)));
     p.halves2 = take(piece(c.group * halves_image_bytes(c.channels, h2, w2)));
@@ -932,10 +972,12 @@ hipError_t launch_conv_tower_prep(hipStream_t s, int cus, const ConvTower &c, co
     p.job[0] = {c.weights[1], base + at.wprep2, reinterpret_cast<float *>(base + at.norms2), c.channels, pad, c.channels};
     p.job[1] = {c.weights[2], base + at.wprep3, reinterpret_cast<float *>(base + at.norms3), c.channels, pad, c.channels};
     p.x = mel;
-    p.count = (uint64_t)c.bins * frames;
+    p.rows = c.bins;
+    p.row_values = p.image_stride = c.chunk_frames;
+    p.row_stride = p.row_limit = frames;
     p.partial = reinterpret_cast<float *>(base + at.partial);
-    p.partials = (uint32_t)std::min<uint64_t>(kMaximaBlocks, (p.count + 255) / 256);
-    conv_prep_kernel<<<2 * pad + p.partials, 256, 0, s>>>(p);
+    p.partials = maxima_blocks(c.bins);
+    conv_prep_kernel<<<2 * pad + c.chunks * p.partials, 256, 0, s>>>(p);
     ConvScaleArgs q{};
     q.partial = p.partial;
     q.partials = p.partials;
@@ -945,7 +987,7 @@ hipError_t launch_conv_tower_prep(hipStream_t s, int cus, const ConvTower &c, co
     q.bias2 = c.bias[1];
     q.channels = c.channels;
     q.scales = reinterpret_cast<float *>(base + at.scales);
-    conv_scale_kernel<<<1, 256, 0, s>>>(q);
+    conv_scale_kernel<<<c.chunks, 256, 0, s>>>(q);
     return hipGetLastError();
 }
 
@@ -953,7 +995,7 @@ hipError_t launch_conv_tower(hipStream_t s, int cus, const ConvTower &c, const f
                              uint32_t count, float *out, void *scratch) {
     uint8_t *base = static_cast<uint8_t *>(scratch);
     const TowerPieces at = tower_pieces(cus, c);
-    const float *scales = reinterpret_cast<const float *>(base + at.scales);
+    const float *scales = reinterpret_cast<const float *>(base + at.scales) + 4 * (size_t)first;
     const uint32_t h1 = (c.bins - 1) / 2 + 1, w1 = (c.chunk_frames - 1) / 2 + 1;
     Conv1HalvesArgs k{};
     k.mel = mel;
@@ -964,11 +1006,11 @@ hipError_t launch_conv_tower(hipStream_t s, int cus, const ConvTower &c, const f
     k.bins = c.bins, k.frames = frames, k.chunk_frames = c.chunk_frames, k.first = first, k.channels = c.channels;
     k.oh = h1, k.ow = w1;
     conv1_halves_kernel<<<dim3((halves_plane(h1, w1).words + 255) / 256, c.channels / kMfIc, count), 256, 0, s>>>(k);
-    ConvMfmaArgs a = mfma_args(base + at.halves1, base + at.wprep2, c.bias[1], scales, c.channels, c.channels, h1, w1);
+    ConvMfmaArgs a = mfma_args(base + at.halves1, base + at.wprep2, c.bias[1], scales, 4, c.channels, c.channels, h1, w1);
     a.halves = base + at.halves2;
     const hipError_t e = launch_mfma<true>(s, cus, a, count, reinterpret_cast<float *>(base + at.part));
     if (e != hipSuccess) return e;
-    ConvMfmaArgs a3 = mfma_args(base + at.halves2, base + at.wprep3, c.bias[2], scales + 2, c.channels, c.channels, a.oh,
+    ConvMfmaArgs a3 = mfma_args(base + at.halves2, base + at.wprep3, c.bias[2], scales + 2, 4, c.channels, c.channels, a.oh,
                                 a.ow);
     a3.out = out;
     return launch_mfma<false>(s, cus, a3, count, reinterpret_cast<float *>(base + at.part));

@@ -60,3 +60,36 @@ def test_conv_non_finite_stays_local(ctx):
     touched[5, 1] = True       # ... and row 10, column 2
     assert np.array_equal(got[:, ~touched], clean[:, ~touched])
     assert np.isnan(got[:, 5, 1]).all() and not (got[:, 2:4, 2:4] == clean[:, 2:4, 2:4]).any()
+
+
+def test_conv_images_of_different_magnitudes(ctx):
+    # An image's result does not depend on the others': each has its own scale.
+    cin, cout, h, w = 32, 64, 13, 11
+    x = normal(6 * cin * h * w, 99, 0).reshape(6, cin, h, w)
+    for i, factor in enumerate((1.0, 1e6, 1e-12, 1e12, 1.0, 1e-30)):
+        x[i] *= np.float32(factor)
+    x[4, 7, 5, 5] = np.float32(1e20)
+    wb = f16_fast(normal(cout * cin * 9, 100, 0, 0.1))
+    b = np.zeros(cout, np.float32)
+    got = run_conv(ctx, x.reshape(-1), wb, b, 6, cout, cin, h, w)
+    for i in (0, 1, 2, 3, 5):
+        want = o.conv3x3s2_gelu(x[i].reshape(-1), wb, b, cout, cin, h, w)
+        assert_close(got[i], want, rtol=1e-5, atol_rms=1e-5, what=f"image {i}")
+        alone = run_conv(ctx, x[i].reshape(-1), wb, b, 1, cout, cin, h, w)
+        assert np.array_equal(got[i], alone[0]), i
+
+
+@pytest.mark.parametrize("outlier", [1e6, 1e9])
+def test_conv_outlier_within_an_image(ctx, outlier):
+    # A value far above its image: the positions that do not read it keep the
+    # 2^-17 that two bf16 terms of each value kept.
+    cin, cout, h, w = 32, 64, 16, 16
+    x = normal(cin * h * w, 101, 0).reshape(cin, h, w)
+    x[3, 5, 5] = np.float32(outlier)
+    wb = f16_fast(normal(cout * cin * 9, 102, 0, 0.1))
+    b = normal(cout, 103, 0, 0.1)
+    got = np.asarray(run_conv(ctx, x.reshape(-1), wb, b, 1, cout, cin, h, w)[0]).reshape(cout, 8, 8)
+    want = np.asarray(o.conv3x3s2_gelu(x.reshape(-1), wb, b, cout, cin, h, w)).reshape(cout, 8, 8)
+    away = np.ones((8, 8), bool)
+    away[2:4, 2:4] = False
+    assert_close(got[:, away], want[:, away], rtol=2e-5, atol_rms=2e-5)

@@ -123,3 +123,27 @@ def test_frontend_against_oracle(ctx, mel_bins, frames, n_window, downsample, d_
         ctx.matrix_release(w.conv_out)
         for b in keep + [mel, enc]:
             b.free()
+
+
+def test_frontend_garbage_stays_in_its_chunk(ctx):
+    # One finite sample of extreme magnitude: the other chunks' rows are what
+    # they are without it.
+    mel_bins, frames, n_window, downsample, d_model = 64, 8 * 5, 4, 64, 128
+    host, w, keep = frontend_weights(ctx, 83, downsample, mel_bins, d_model, o.Q8)
+    log_mel = normal(mel_bins * frames, 84).reshape(mel_bins, frames)
+    outputs = []
+    enc = ctx.buffer(5 * d_model * 4)
+    try:
+        for value in (log_mel[9, 19], np.float32(1e20)):
+            log_mel[9, 19] = value
+            mel = ctx.to_device(log_mel)
+            assert ctx.audio_frontend(w, mel.ptr, mel_bins, frames, n_window, downsample, d_model, enc.ptr, 5) == 5
+            outputs.append(enc.download(np.float32).reshape(5, d_model).copy())
+            mel.free()
+    finally:
+        ctx.matrix_release(w.conv_out)
+        for b in keep + [enc]:
+            b.free()
+    others = [0, 1, 3, 4]
+    assert np.array_equal(outputs[0][others], outputs[1][others])
+    assert not np.array_equal(outputs[0][2], outputs[1][2])
