@@ -582,7 +582,8 @@ int32_t plan_step(qwh_decoder *d) {
     }
     d->batched = batch_form;
     const bool per_token_q4 = q4_fused && !batch_form;
-    d->fold_embed = per_token_q4 && first.qkv.format == QWH_FORMAT_Q4 &&
+    // (The GEMV decodes quantized embedding rows; f32 / f16 tables are embed_kernel's.)
+    d->fold_embed = per_token_q4 && first.qkv.format == QWH_FORMAT_Q4 && !is_dense_format(d->embed.format) &&
                     gemv_q4_source_supported(GemvInput::Embed, first.qkv.rows, first.qkv.cols);
     d->fold_argmax = per_token_q4 && !d->head_batched && d->lm_head.format == QWH_FORMAT_Q4;
     d->split_parts = false;

@@ -149,6 +149,39 @@ def test_matrices_rebound_in_another_format(ctx):
         ref.close()
 
 
+@pytest.mark.parametrize("fmt", [o.F16, o.F32])
+@pytest.mark.parametrize("batch", [1, 2, 3, 8, 9])
+def test_q4_layers_with_an_unquantized_embedding(ctx, fmt, batch):
+    # decoder.zig:346-360 embeddingRow's f32 / f16 arms under q4 layers: the
+    # oracle takes the same row as given (forward_row). An f32 cache: a q8 row's
+    # code near a tie may fall either way, which the next step sees.
+    seed, c = 37, TINY
+    values = o.normal(c["vocab"] * c["hidden"], seed, 77, 0.02).reshape(c["vocab"], c["hidden"])
+    elements = values.astype(np.float16).view(np.uint16) if fmt == o.F16 else values
+    gpu = qa.Decoder(ctx, batch=batch, cache_format=o.CACHE_F32, **c)
+    ref = o.Decoder(seed, batch, o.Q4, o.CACHE_F32, **c)
+    handle = None
+    try:
+        gpu.init_synthetic(seed)
+        handle = ctx.matrix_upload(fmt, c["vocab"], c["hidden"], None, elements.reshape(-1))
+        gpu.set_matrix(qa.T_EMBED, 0, handle)
+        for b in range(batch):
+            gpu.prefill_random(b, 3 + b, seed)
+            ref.prefill_random(b, 3 + b)
+        for step in range(3):
+            tokens = [(step * 71 + b * 13 + 5) % c["vocab"] for b in range(batch)]
+            gpu.forward(tokens, True)
+            for b in range(batch):
+                row = o.embedding_row(fmt, None, elements, c["vocab"], c["hidden"], tokens[b])
+                ref.forward_row(b, tokens[b], row, True)
+                assert_close(gpu.logits(b), ref.logits(b), rtol=1e-4, atol_rms=1e-4, what=f"step {step} seq {b}")
+    finally:
+        if handle is not None:
+            ctx.matrix_release(handle)
+        gpu.close()
+        ref.close()
+
+
 def oracle_until(ref, b, token, max_tokens, stops):
     """wasm/model.zig:423-451 decodeStep looped to the end of the sequence."""
     emitted = []
