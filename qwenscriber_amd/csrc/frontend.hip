@@ -309,6 +309,13 @@ __global__ __launch_bounds__(256, NT == 1 && R <= 6 ? 3 : 2) void conv3x3s2_gelu
         }
     }
     __builtin_amdgcn_s_waitcnt(kConvWait<0>);  // (the last copy, unused, before the LDS is given back)
+    // (The last stage loaded weights that nothing multiplies: a use, or a
+    // compiler that takes that stage out of the loop may drop them from under
+    // the waits that count them.)
+#pragma unroll
+    for (int tap = 0; tap < 9; ++tap)
+#pragma unroll
+        for (int i = 0; i < 2; ++i) asm volatile("" ::"v"(__builtin_bit_cast(cu4, wa[tap][i])));
     if (oc0 >= a.out_ch) return;
     // (Computed again: no register of the loop's, at its limit, holds them.)
     const int out_lane = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)), out_half = out_lane >> 5;

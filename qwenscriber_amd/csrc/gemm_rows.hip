@@ -338,6 +338,16 @@ __device__ __forceinline__ void rows_block(const RowsArgs &a, uint32_t row_block
             static_for<CG>([&](auto at) __attribute__((always_inline)) {
                 if (gc + decltype(at)::value < g1) step(at, std::true_type{}, gc);
             });
+        } else {
+            // (The last chunk's step loaded weights that nothing multiplies: a
+            // use, or a compiler that takes that step out of the loop may drop
+            // them from under the waits that count them.)
+#pragma unroll
+            for (int i = 0; i < CG; ++i)
+#pragma unroll
+                for (int k = 0; k < CW; ++k) asm volatile("" ::"v"(rw[i][k]));
+#pragma unroll
+            for (int i = 0; i < CG / 2; ++i) asm volatile("" ::"v"(rs[i]));
         }
     }
 
