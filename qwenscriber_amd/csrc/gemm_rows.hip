@@ -271,7 +271,13 @@ __device__ __forceinline__ void rows_block(const RowsArgs &a, uint32_t row_block
         // its way: vector memory completes in order), in every wavefront
         // after the barrier; the buffer refilled now was last read before it.
         // No weights follow the last chunk (the compiler would drop loads that
-        // nothing uses, and a count that expects them would not wait).
+        // nothing uses, and a count that expects them would not wait). In the
+        // two-group chunks of q5 and q8 the codes taken at i == 0 are awaited
+        // by the compiler's own wait, which with copies to LDS in flight is
+        // for everything: once a chunk nothing travels. Counting PT there
+        // keeps the next words in flight: 4096 x 2048 q8 at 402 tokens 34.9 ->
+        // 31.2 us, where a CU has one workgroup, but 2048 x 6144 43.0 -> 44.1
+        // and 896 x 7680 34.1 -> 35.7, where it has two.
         constexpr int after = PT + (ahead && (i == 1 || i == 2 || CG == 2) ? WL : 0);
         __builtin_amdgcn_s_waitcnt(kWait<after>);
         __builtin_amdgcn_s_barrier();
