@@ -104,6 +104,10 @@ def frontend_weights(ctx, seed, downsample, mel_bins, d_model, fmt):
     (32, 19, 4, 16, 64, o.Q8),         # ragged third chunk of 3 frames, q8 projection
     (64, 8, 4, 64, 128, o.Q5),         # exactly one chunk, q5 projection
     (128, 250, 50, 480, 896, o.F16),   # the 0.6B shape with an f16 projection (7680-wide rows)
+    (128, 95, 50, 480, 896, o.Q4),     # one chunk: conv2 and conv3 with their stages split over workgroups
+    (128, 199, 50, 480, 896, o.Q8),    # two: fewer slices
+    (128, 650, 50, 480, 896, o.Q4),    # seven: conv2 on 64-position workgroups
+    (32, 8 * 34 + 3, 4, 32, 64, o.Q8), # 35: the second run of chunks in the first's buffers, the last one ragged
 ])
 def test_frontend_against_oracle(ctx, mel_bins, frames, n_window, downsample, d_model, fmt):
     host, w, keep = frontend_weights(ctx, 81, downsample, mel_bins, d_model, fmt)
