@@ -168,10 +168,8 @@ bool gemv_b8_supported(int format, uint32_t rows, uint32_t cols);
 hipError_t launch_gemv_b8(hipStream_t s, int cus, const GemvInput &in, const Matrix &w, uint32_t tokens,
                           float *out, const float *residual);
 // A few tokens (at least 2) of a matrix this small run faster as one launch
-// of the per-token GEMV than on the matrix cores; likewise the products of a
-// decoder layer of `weights` values in all.
+// of the per-token GEMV than on the matrix cores (gemv_plan.h).
 bool gemv_tokens_preferred(const Matrix &w, uint32_t tokens);
-bool gemv_tokens_preferred_layer(int format, uint64_t weights, uint32_t tokens);
 hipError_t launch_gemv_tokens(hipStream_t s, int cus, const GemvInput &in, const Matrix &w, uint32_t tokens,
                               float *out);
 hipError_t launch_gemv_q8(hipStream_t s, int cus, const float *x, const Matrix &w,

@@ -36,6 +36,7 @@
 
 #include "common.h"
 #include "device.h"
+#include "gemv_plan.h"
 
 namespace qwh {
 namespace {
@@ -573,10 +574,9 @@ int32_t plan_step(qwh_decoder *d) {
     // (with every q4 one forming its own activations), the long lm_head still
     // on the matrix cores.
     const qwh_decoder::Layer &first = d->layers[0];
-    uint64_t weights = 0;
-    for (const Matrix *m : {&first.qkv, &first.o, &first.gu, &first.down}) weights += (uint64_t)m->rows * m->cols;
+    const Matrix *const products[] = {&first.qkv, &first.o, &first.gu, &first.down};
     d->head_batched = batch_form;
-    if (batch_form && q4_fused && gemv_tokens_preferred_layer(first.gu.format, weights, d->batch)) {
+    if (batch_form && q4_fused && plan::token_gemv_layer(products, 4, d->batch)) {
         batch_form = false;
         d->head_batched = !gemv_tokens_preferred(d->lm_head, d->batch);
     }

@@ -41,6 +41,7 @@
 
 #include "common.h"
 #include "device.h"
+#include "gemv_plan.h"
 
 namespace qwh {
 namespace {
@@ -1656,46 +1657,24 @@ hipError_t launch_gemv_b8(hipStream_t s, int cus, const GemvInput &in, const Mat
                : dispatch_b8<Fmt8::Q8, Src::F32>(s, cus, args, tokens);
 }
 
-// One launch that reads the matrix once per token, mostly from the caches,
-// against the matrix-core form's three (activation digits, product, slice
-// sum): 2 tokens of q8 1024 x 3072 4.1 us against 9.4. The reads and the
-// activation encoding grow with the tokens; the two meet (us, this form /
-// matrix cores) for q4 at 6144 x 1024 and 16 tokens 8.9 / 9.5, 12288 x 2048 at
-// 4 and 6 9.2 / 11.5 and 12.3 / 11.8, 2048 x 6144 at 6 9.9 / 10.0; for q8 at
-// 4096 x 2048 and 8 8.4 / 9.2, 12288 x 2048 at 2 and 3 9.5 / 11.5 and 12.8 /
-// 11.6, 2048 x 6144 at 3 and 4 8.6 / 10.3 and 10.5 / 10.2; for q5 at 6144 x
-// 1024 and 8 7.9 / 9.3 and 10 9.9 / 9.4, 2048 x 6144 at 3 8.9 / 10.4.
 bool gemv_tokens_preferred(const Matrix &w, uint32_t tokens) {
-    if (tokens < 2) return false;
-    const uint64_t work = (uint64_t)w.rows * w.cols * tokens;
-    const bool wide = w.cols > 3072;  // (longer rows: more encoding per workgroup)
     switch (w.format) {
     case QWH_FORMAT_Q4:
-        return tokens <= 16 && work <= (wide ? 64000000u : 105000000u) && gemv_q4_fused_supported(w.rows, w.cols);
+        if (!gemv_q4_fused_supported(w.rows, w.cols)) return false;
+        break;
     case QWH_FORMAT_Q5:
-        return tokens <= 12 && work <= (wide ? 40000000u : 50400000u) && gemv_b8_supported(w.format, w.rows, w.cols);
     case QWH_FORMAT_Q8:
-        return tokens <= 12 && work <= (wide ? 40000000u : 70000000u) && gemv_b8_supported(w.format, w.rows, w.cols);
+        if (!gemv_b8_supported(w.format, w.rows, w.cols)) return false;
+        break;
     default: return false;
     }
+    return plan::token_gemv(w.format, w.rows, w.cols, tokens);
 }
 
 hipError_t launch_gemv_tokens(hipStream_t s, int cus, const GemvInput &in, const Matrix &w, uint32_t tokens,
                               float *out) {
     if (w.format == QWH_FORMAT_Q4) return launch_gemv_q4_src(s, cus, in, w, tokens, out, nullptr);
     return launch_gemv_b8(s, cus, in, w, tokens, out, nullptr);
-}
-
-// Six launches a layer against nine. Four steps (ms, this form / matrix
-// cores): q4 0.6B (15.7M weights a layer) at 3 and 8 sequences 3.51 / 5.18 and
-// 4.59 / 5.67, 1.7B (50.3M) at 5 and 7 5.88 / 6.19 and 7.15 / 6.39; q8 0.6B at
-// 8 5.58 / 5.83, 1.7B at 3 and 4 6.25 / 6.43 and 7.28 / 6.50; q5 1.7B at 3 and
-// 4 5.81 / 6.39 and 6.77 / 6.46. Two sequences would gain most (3.29 / 4.99)
-// but keep the products of a short prompt, value for value: a prompt's cache
-// rows equal those of its tokens stepped one by one there.
-bool gemv_tokens_preferred_layer(int format, uint64_t weights, uint32_t tokens) {
-    return tokens >= 3 && tokens <= 8 &&
-           weights * tokens <= (format == QWH_FORMAT_Q4 ? 255000000ull : 155000000ull);
 }
 
 }  // namespace qwh

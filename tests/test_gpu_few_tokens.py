@@ -21,6 +21,10 @@ SMALL = dict(hidden=256, layers=2, heads=4, kv_heads=2, head_dim=128, ffn=512, m
     (qa.FORMAT_Q5, 3255, 6144, 2), (qa.FORMAT_Q5, 8203, 3072, 2), (qa.FORMAT_Q5, 33000, 512, 3),
     (qa.FORMAT_Q8, 1, 64, 2), (qa.FORMAT_Q8, 33, 192, 12), (qa.FORMAT_Q8, 33, 192, 13),
     (qa.FORMAT_Q8, 1024, 3072, 2), (qa.FORMAT_Q8, 3255, 6144, 2), (qa.FORMAT_Q8, 31, 6208, 2),  # past the GEMV's rows
+    # A wavefront a row: few rows x tokens there, more on the matrix cores.
+    (qa.FORMAT_Q5, 3584, 896, 4), (qa.FORMAT_Q5, 3584, 896, 6), (qa.FORMAT_Q5, 12288, 128, 12),
+    (qa.FORMAT_Q8, 3584, 896, 4), (qa.FORMAT_Q8, 3584, 896, 6), (qa.FORMAT_Q8, 12288, 128, 12),
+    (qa.FORMAT_Q8, 1027, 2560, 8), (qa.FORMAT_Q8, 1027, 2560, 11),
 ])
 def test_linear_few_tokens(ctx, fmt, rows, cols, tokens):
     _, scales, data = quantized_matrix(fmt, rows, cols, 3, rows)
