@@ -453,7 +453,11 @@ int32_t qwh_linear(qwh_ctx *ctx, uint64_t matrix, const float *x_dev, uint32_t c
     QWH_TRY(check_device_ptr(ctx, out_dev, "out"));
     if (((uintptr_t)x_dev & 15u) != 0) return fail(ctx, QWH_E_INVALID_ARGUMENT, "x must be 16-byte aligned");
     if (m->rows == 0) return QWH_OK;
-    if (gemv_tokens_preferred(*m, tokens)) {
+    // (In place, x must be read before the first result is stored, as the forms
+    // with an activation pass do.)
+    const uintptr_t x_at = (uintptr_t)x_dev, out_at = (uintptr_t)out_dev;
+    const bool in_place = x_at < out_at + sizeof(float) * tokens * m->rows && out_at < x_at + sizeof(float) * tokens * cols;
+    if (!in_place && gemv_tokens_preferred(*m, tokens)) {
         GemvInput in;
         in.mode = GemvInput::F32;
         in.x = x_dev;

@@ -37,6 +37,22 @@ def test_linear_few_tokens(ctx, fmt, rows, cols, tokens):
     ctx.matrix_release(m)
 
 
+@pytest.mark.parametrize("fmt", [qa.FORMAT_Q4, qa.FORMAT_Q5, qa.FORMAT_Q8])
+@pytest.mark.parametrize("tokens,offset", [(2, 0), (12, 0), (4, 512)])
+def test_linear_few_tokens_in_place(ctx, fmt, tokens, offset):
+    # The result over x, or over a part of it: every row is read before any is
+    # written.
+    rows = cols = 1024
+    _, scales, data = quantized_matrix(fmt, rows, cols, 13, 0)
+    x = normal(tokens * cols, 14, tokens)
+    want = o.linear_quantized(fmt, scales, data, rows, cols, x, tokens)
+    m = ctx.matrix_upload(fmt, rows, cols, scales, data)
+    buf = ctx.to_device(np.concatenate([x, np.zeros(offset, np.float32)]))
+    ctx.linear(m, buf.ptr, cols, tokens, buf.ptr + 4 * offset)
+    assert_close(buf.download(np.float32)[offset:offset + tokens * rows], np.asarray(want).reshape(-1), rtol=1e-4, atol_rms=1e-5)
+    ctx.matrix_release(m)
+
+
 @pytest.mark.parametrize("fmt", [o.Q4, o.Q5, o.Q8])
 @pytest.mark.parametrize("batch,vocab", [
     (3, 500), (8, 500),      # layers and lm_head per token
