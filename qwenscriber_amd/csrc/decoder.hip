@@ -1441,10 +1441,12 @@ enum class PrefillForm { MatrixCores, Rows, Positions };
 
 // The rows from which a MatrixCores chunk runs on the 32-token tiles of the
 // f16 matrix cores (prefill_chunk_gemm) rather than the 16-token ones, by the
-// layers' shapes; ~0u: never. The two meet near 6e9 multiply-adds a layer: a
-// 1.7B decoder's prompt (50.3M weights a layer) took 2.96 ms with 16-token
-// tiles and 3.06 with these at 128 positions, 3.85 and 3.72 at 192; a 0.6B
-// one's (15.7M) 2.91 and 3.03 at 256, 5.27 and 4.12 at 402.
+// layers' shapes; ~0u: never. The two meet near 6e9 multiply-adds a layer, and
+// not below five tiles (ms, 16-token tiles / these): a 1.7B decoder's prompt
+// (50.3M weights a layer), q4 2.90 / 3.05 at 120 positions and 2.94 / 2.99 at
+// 128, 3.28 / 3.22 at 135, 3.52 / 3.29 at 160, 4.81 / 4.11 at 256; a 0.6B one's
+// (15.7M), q4 3.66 / 3.80 at 382, 3.93 / 3.84 at 392, 4.17 / 4.07 at 432, q8
+// 3.88 / 3.95 and 4.19 / 4.05, q5 3.96 / 4.20, 4.26 / 4.27 and 4.55 / 4.50.
 uint32_t gemm_rows_from(const qwh_decoder *d) {
     const qwh_decoder::Layer &L = d->layers[0];
     uint64_t weights = 0;
@@ -1452,7 +1454,7 @@ uint32_t gemm_rows_from(const qwh_decoder *d) {
         if (m->cols < 256 || m->cols > 8192) return ~0u;
         weights += (uint64_t)m->rows * m->cols;
     }
-    const uint64_t rows = (6000000000ull + weights - 1) / weights;
+    const uint64_t rows = std::max<uint64_t>(129, (6000000000ull + weights - 1) / weights);
     return rows > kPrefillChunk ? ~0u : (uint32_t)rows;
 }
 
