@@ -258,7 +258,7 @@ struct RowsOutput {
     float *partials = nullptr;          // rows_partial_bytes, needed for a K split
 };
 bool gemm_rows_supported(const Matrix &w);
-// The form is the faster one for this many tokens.
+// The form is the faster one for this many tokens (rows_plan.h).
 bool gemm_rows_preferred(const Matrix &w, uint32_t tokens);
 size_t rows_activation_bytes(uint32_t tokens, uint32_t cols);
 size_t rows_partial_bytes(int cus, uint32_t tokens, const Matrix &w);

@@ -43,6 +43,7 @@
 
 #include "common.h"
 #include "device.h"
+#include "rows_plan.h"
 
 namespace qwh {
 namespace {
@@ -52,7 +53,10 @@ typedef _Float16 h8 __attribute__((ext_vector_type(8)));
 typedef float f16x __attribute__((ext_vector_type(16)));
 typedef uint32_t u4 __attribute__((ext_vector_type(4)));
 
-constexpr int kTile = 32;                              // tokens, and weight rows, of one MFMA tile
+using plan::RowsPlan;
+using plan::rows_plan;
+
+constexpr int kTile = plan::kRowsTile;                 // tokens, and weight rows, of one MFMA tile
 constexpr int kStepBytes = 2 * 64 * 16;                // hi and lo of one step
 constexpr int kGroupPieces = 4 * kStepBytes / 16;      // 16-byte words of a (tile, group)
 
@@ -402,7 +406,7 @@ __device__ __forceinline__ void rows_block(const RowsArgs &a, uint32_t row_block
 // the eight dies in turn, so a die takes whole (row block, slice) units and
 // walks their token blocks: a weight line is fetched into one die's L2, and
 // with as many slices as dies a die reads one slice of the activations.
-constexpr uint32_t kDies = 8;
+using plan::kDies;
 
 template <Codes C, int W, int TT>
 __global__ __launch_bounds__(64 * W, 2) void gemm_rows_kernel(const RowsArgs a) {
@@ -658,50 +662,7 @@ size_t uneven_bytes(uint32_t tokens, uint32_t cols) {
     return (size_t)((tokens + kTile - 1) / kTile) * kTile * (cols / 64) * sizeof(float);
 }
 
-constexpr int kWaves = 4;
-
-struct RowsPlan {
-    int token_tiles = 1;  // per workgroup
-    uint32_t slices = 1, slice_groups = 0;
-};
-
-// One group step of a CU that holds `per_cu` workgroups (us), as sweeps of
-// shapes from 896 x 896 to 12288 x 2048 at 64 to 1024 tokens measured it: a
-// CU's first workgroup waits for its own loads and barriers, which more of
-// them hide.
-float step_us(int token_tiles, uint32_t per_cu) {
-    if (token_tiles == 2) return per_cu == 1 ? 0.76f : per_cu == 2 ? 1.13f : 0.53f * (float)per_cu;
-    return per_cu == 1 ? 0.62f : per_cu == 2 ? 0.77f : 0.38f * (float)per_cu;
-}
-
-// Token tiles per workgroup and K slices by the least estimated time; a split
-// writes its partial sums and reads them back, in a launch of its own unless
-// the caller's next pass adds them (`folded`).
-RowsPlan rows_plan(int cus, uint32_t tokens, uint32_t rows, uint32_t cols, uint32_t max_slices, bool folded) {
-    const uint32_t groups = cols / 64, tiles = (tokens + kTile - 1) / kTile;
-    const uint32_t row_blocks = (rows + kWaves * kTile - 1) / (kWaves * kTile);
-    RowsPlan best;
-    best.slice_groups = groups;
-    float least = 0.0f;
-    for (int tt = 1; tt <= 2; ++tt)
-        for (uint32_t want = 1; want <= max_slices; ++want) {
-            RowsPlan p;
-            p.token_tiles = tt;
-            // Slices of whole weight chunks, none empty.
-            p.slice_groups = ((groups + want - 1) / want + 3) & ~3u;
-            p.slices = (groups + p.slice_groups - 1) / p.slice_groups;
-            if (p.slices != want) continue;
-            // The fullest die's share.
-            const uint64_t units = ((uint64_t)row_blocks * p.slices + kDies - 1) / kDies;
-            const uint64_t die_cus = std::max(1u, (uint32_t)cus / kDies);
-            const uint32_t per_cu = (uint32_t)((units * ((tiles + tt - 1) / tt) + die_cus - 1) / die_cus);
-            float us = (float)std::min(p.slice_groups, groups) * step_us(tt, per_cu);
-            if (p.slices > 1)
-                us += (folded ? 0.5f : 3.0f) + (float)p.slices * (float)(tiles * kTile) * (float)rows * 8.0f / 4.5e6f;
-            if (least == 0.0f || us < least) least = us, best = p;
-        }
-    return best;
-}
+constexpr int kWaves = plan::kRowsWaves;
 
 template <Codes C>
 void launch_rows(hipStream_t s, const RowsPlan &plan, const RowsArgs &a) {
@@ -718,15 +679,8 @@ bool gemm_rows_supported(const Matrix &w) {
            w.cols >= 256 && w.rows != 0;
 }
 
-// The 16-token tiles (gemv_batch.hip) take less fixed time: their activation
-// pass needs no whole row, and more and smaller workgroups fill the device.
-// Both sides, f32 rows in and out (us, 16-token tiles against these): 896 x
-// 896 at 402 tokens 10.9 / 15.3, 2048 x 2048 at 256 19.0 / 19.7, 896 x 7680 at
-// 192 24.3 / 25.4 and at 402 41.0 / 36.3, 4096 x 2048 at 192 27.4 / 27.2, 2048
-// x 6144 at 96 23.2 / 25.4 and at 128 27.0 / 23.1, 12288 x 2048 at 96 30.7 /
-// 32.0 and at 402 90.1 / 57.7. They meet near 1.6e9 multiply-adds.
 bool gemm_rows_preferred(const Matrix &w, uint32_t tokens) {
-    return gemm_rows_supported(w) && tokens >= 128 && (uint64_t)w.rows * w.cols * tokens >= 1600000000ull;
+    return gemm_rows_supported(w) && plan::rows_preferred(w.format, w.rows, w.cols, tokens);
 }
 
 size_t rows_activation_bytes(uint32_t tokens, uint32_t cols) {

@@ -2,12 +2,13 @@
 // built with g++ only: for every shape and form the decoder step, the
 // prefill and the attention entry points launch, the bytes they allocate
 // (sized before the launch form is known) hold the records of the ranges
-// the launch then writes. And of the few-token products' rule (gemv_plan.h)
-// against measured pairs. Exit status 0 when every case holds.
+// the launch then writes. And of the products' rules (gemv_plan.h,
+// rows_plan.h) against measured pairs. Exit status 0 when every case holds.
 #include <cstdio>
 
 #include "../csrc/attention_plan.h"
 #include "../csrc/gemv_plan.h"
+#include "../csrc/rows_plan.h"
 
 using qwh::AttentionArgs;
 namespace plan = qwh::plan;
@@ -45,7 +46,7 @@ void check(const char *who, int cus, const AttentionArgs &a, bool decoder, size_
 struct Pair {
     int format;
     uint32_t rows, cols, tokens;
-    float per_token, matrix_cores;
+    float first, second;  // us: the form that the rule takes where it is faster, and the other
 };
 
 const Pair pairs[] = {
@@ -100,10 +101,10 @@ void check_token_gemv() {
     for (const Pair &p : pairs) {
         const bool takes = plan::token_gemv(p.format, p.rows, p.cols, p.tokens);
         ++cases;
-        if (takes == (p.per_token < p.matrix_cores)) continue;
+        if (takes == (p.first < p.second)) continue;
         ++failures;
         std::printf("FAIL few tokens: format %d %u x %u, %u tokens: per token %.1f us, matrix cores %.1f, rule %d\n", p.format,
-                    p.rows, p.cols, p.tokens, p.per_token, p.matrix_cores, (int)takes);
+                    p.rows, p.cols, p.tokens, p.first, p.second, (int)takes);
     }
     // A layer's matrices count by their own formats: 0.6B shapes, 8 sequences,
     // with q4 or q8 products; the 1.7B's at 3 and 5 with its down product in
@@ -130,10 +131,48 @@ void check_token_gemv() {
     }
 }
 
+// Many tokens' product: the 32-token tiles, and the 16-token ones.
+const Pair many[] = {
+    {QWH_FORMAT_Q4, 2048, 2048, 402, 26.4f, 27.8f},
+    {QWH_FORMAT_Q8, 2048, 2048, 402, 28.1f, 29.9f},
+    {QWH_FORMAT_Q4, 2048, 2048, 512, 27.7f, 30.7f},
+    {QWH_FORMAT_Q8, 4096, 2048, 224, 26.9f, 30.0f},
+    {QWH_FORMAT_Q4, 2048, 6144, 128, 23.7f, 26.1f},
+    {QWH_FORMAT_Q5, 2048, 6144, 160, 32.4f, 33.1f},
+    {QWH_FORMAT_Q8, 6144, 1024, 256, 20.2f, 22.6f},
+    {QWH_FORMAT_Q4, 4096, 1024, 402, 20.1f, 22.6f},
+    {QWH_FORMAT_Q5, 3584, 896, 512, 21.9f, 25.7f},
+    {QWH_FORMAT_Q8, 896, 7680, 256, 29.6f, 30.7f},
+    {QWH_FORMAT_Q4, 1024, 6144, 256, 25.1f, 27.1f},
+    {QWH_FORMAT_Q8, 2048, 3072, 256, 25.3f, 27.4f},
+    {QWH_FORMAT_Q5, 3000, 2560, 224, 27.2f, 30.9f},
+    {QWH_FORMAT_Q8, 8191, 1024, 224, 22.9f, 27.7f},
+    {QWH_FORMAT_Q4, 12288, 2048, 128, 27.2f, 36.0f},
+    {QWH_FORMAT_Q4, 33, 1088, 44600, 186.2f, 126.9f},
+    {QWH_FORMAT_Q5, 33, 1088, 44600, 196.2f, 636.5f},
+    {QWH_FORMAT_Q8, 100, 6144, 4000, 71.7f, 65.3f},
+    {QWH_FORMAT_Q4, 300, 4096, 3000, 61.0f, 57.8f},
+    {QWH_FORMAT_Q8, 200, 8128, 1000, 38.6f, 85.0f},
+    {QWH_FORMAT_Q4, 1600, 7808, 129, 28.0f, 57.6f},
+    {QWH_FORMAT_Q8, 1480, 8256, 131, 35.7f, 44.2f},
+};
+
+void check_rows() {
+    for (const Pair &p : many) {
+        const bool takes = plan::rows_preferred(p.format, p.rows, p.cols, p.tokens);
+        ++cases;
+        if (takes == (p.first < p.second)) continue;
+        ++failures;
+        std::printf("FAIL many tokens: format %d %u x %u, %u tokens: 32-token tiles %.1f us, 16-token %.1f, rule %d\n", p.format,
+                    p.rows, p.cols, p.tokens, p.first, p.second, (int)takes);
+    }
+}
+
 }  // namespace
 
 int main() {
     check_token_gemv();
+    check_rows();
     // The Qwen3-ASR decoders (0.6B: 16 / 8 heads of 128; 1.7B the same
     // heads), the test suites' shapes, and every head layout the kernels
     // are built for.

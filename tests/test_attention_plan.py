@@ -7,7 +7,7 @@ decoder at create, the prefill per chunk, the attention entry points) hold
 the records of every range the launch then writes. A buffer sized for the
 plain form's ranges but launched in the decoder form is the fault this pins
 (its range records ran past the buffer's end). The same program holds the
-few-token products' rule (gemv_plan.h) to measured pairs of its two forms."""
+rules of the products' forms (gemv_plan.h, rows_plan.h) to measured pairs."""
 import os
 import shutil
 import subprocess

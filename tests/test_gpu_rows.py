@@ -57,7 +57,8 @@ def error_bound(x, w):
     (2048, 6144, 160),   # K split over slices
     (1600, 7808, 129),   # 122 groups in slices of whole chunks, the last one short
     (1480, 8256, 131),   # past the activation pass's registers (129 groups)
-    (33, 1088, 44600),   # one row past a tile
+    (33, 1088, 44600),   # one row past a tile (q5; q4 and q8 on 16-token tiles)
+    (513, 1088, 2900),   # one row past a workgroup's
 ])
 def test_linear_many_tokens(ctx, fmt, rows, cols, tokens):
     if fmt == qa.FORMAT_Q5 and cols == 8256:
