@@ -449,11 +449,12 @@ struct ConvWeightsJob {
 
 struct ConvPrepArgs {
     ConvWeightsJob job[2];
-    // Row r of image b: x + b * image_stride + r * row_stride, row_values
-    // values, of which those below row_limit - b * image_stride exist.
+    // Row r of image b: x + b * image_stride + r * row_stride, at most
+    // row_values values: what is left of `limit` after b * image_used + r *
+    // row_used of it.
     const float *x;
-    uint64_t image_stride, row_stride, row_limit, row_values;
-    uint32_t rows;
+    uint64_t image_stride, row_stride, limit, image_used, row_used;
+    uint32_t rows, row_values;
     float *partial;              // [image][partials]
     uint32_t partials;
 };
@@ -469,17 +470,23 @@ __global__ __launch_bounds__(256) void conv_prep_kernel(const ConvPrepArgs a) {
     const bool maxima = block >= a.job[0].oc_pad + a.job[1].oc_pad;
     if (maxima) {
         block -= a.job[0].oc_pad + a.job[1].oc_pad;
-        const uint64_t first = block / a.partials * a.image_stride;
-        const uint64_t n = min(a.row_values, a.row_limit - first);
-        // (Four rows' loads at a time; past the last row, that row again.)
+        const uint64_t image = block / a.partials;
+        // (Four rows' loads at a time; past the last row, that row again, and
+        // past a row's end its last value.)
         for (uint32_t r = (block % a.partials * 4 + (threadIdx.x >> 6)) * 4; r < a.rows; r += a.partials * 16) {
             const float *row[4];
+            uint32_t last[4], longest = 0;
 #pragma unroll
-            for (uint32_t k = 0; k < 4; ++k) row[k] = a.x + first + min(r + k, a.rows - 1) * a.row_stride;
-            for (uint64_t i = threadIdx.x & 63; i < n; i += 64) {
+            for (uint32_t k = 0; k < 4; ++k) {
+                const uint64_t at = min(r + k, a.rows - 1);
+                row[k] = a.x + image * a.image_stride + at * a.row_stride;
+                last[k] = (uint32_t)min((uint64_t)a.row_values, a.limit - image * a.image_used - at * a.row_used) - 1;
+                longest = max(longest, last[k]);
+            }
+            for (uint32_t i = threadIdx.x & 63; i <= longest; i += 64) {
                 float m[4];
 #pragma unroll
-                for (int k = 0; k < 4; ++k) m[k] = fabsf(row[k][i]);
+                for (int k = 0; k < 4; ++k) m[k] = fabsf(row[k][min(i, last[k])]);
 #pragma unroll
                 for (int k = 0; k < 4; ++k) v = m[k] < __builtin_inff() ? fmaxf(v, m[k]) : v;
             }
@@ -529,19 +536,25 @@ __global__ __launch_bounds__(256) void conv_prep_kernel(const ConvPrepArgs a) {
         *to = maxima ? fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3])) : (red[0] + red[1]) + (red[2] + red[3]);
 }
 
-// An image's scales {2^e, 2^-e} from bounds on its magnitudes, one workgroup
-// an image: the first from the partial maxima of the input -- that input
-// itself, or (conv1) the result of a one-channel convolution of it -- and the
-// next from the first's bound through a convolution's weight sums: |gelu(y)|
-// <= |y| <= |bias| + sum |w| * bound. (A bound a thousand times the largest
-// value still keeps it to 2^-41.)
+// An image's scales {2^e, 2^-e} for magnitudes to m, with room for the bound's
+// own rounding.
+__device__ __forceinline__ float2 scale_of(float m) {
+    const int e = dev::chunk_exponent(fminf(m * 1.01f, 3.4e38f));
+    return make_float2(__builtin_ldexpf(1.0f, 15 - e), __builtin_ldexpf(1.0f, e - 15));
+}
+
+// The scales of the tower's intermediate tensors from bounds on their
+// magnitudes, one workgroup a chunk: the first, of conv1's result, from the
+// partial maxima of the chunk through conv1's weight sums, the second from the
+// first's bound through conv2's: |gelu(y)| <= |y| <= |bias| + sum |w| * bound.
+// (A bound a thousand times the largest value still keeps it to 2^-41.)
 struct ConvScaleArgs {
     const float *partial;
     uint32_t partials;
-    const uint16_t *conv1;       // [channels][9] f16 bits, or null
-    const float *bias1, *norms2, *bias2;  // norms2 null: the first scale only
+    const uint16_t *conv1;       // [channels][9] f16 bits
+    const float *bias1, *norms2, *bias2;
     uint32_t channels;
-    float *scales;               // per image, {s, 1 / s} of the first, then (norms2) of the next
+    float *scales;               // per chunk, {s, 1 / s} of the first, then of the second
 };
 
 __device__ __forceinline__ float block_max_256(float v, float *red) {
@@ -556,41 +569,42 @@ __global__ __launch_bounds__(256) void conv_scale_kernel(const ConvScaleArgs a) 
     __shared__ float red[4];
     float v = 0.0f;
     for (uint32_t i = threadIdx.x; i < a.partials; i += 256) v = fmaxf(v, a.partial[(size_t)blockIdx.x * a.partials + i]);
-    float *scales = a.scales + (size_t)blockIdx.x * (a.norms2 ? 4 : 2);
     float bound = block_max_256(v, red);
-    auto emit = [&](float m, float *to) {
-        // 2^e > m, with room for the bound's own rounding.
-        const int e = dev::chunk_exponent(fminf(m * 1.01f, 3.4e38f));
-        if (threadIdx.x == 0) to[0] = __builtin_ldexpf(1.0f, 15 - e), to[1] = __builtin_ldexpf(1.0f, e - 15);
-    };
-    if (a.conv1) {
-        v = 0.0f;
-        for (uint32_t c = threadIdx.x; c < a.channels; c += 256) {
-            float sum = 0.0f;
-            for (int k = 0; k < 9; ++k) sum += fabsf(dev::f16_bits_to_f32(a.conv1[(size_t)c * 9 + k]));
-            v = fmaxf(v, fabsf(a.bias1[c]) + sum * bound);
-        }
-        bound = block_max_256(v, red);
+    v = 0.0f;
+    for (uint32_t c = threadIdx.x; c < a.channels; c += 256) {
+        float sum = 0.0f;
+        for (int k = 0; k < 9; ++k) sum += fabsf(dev::f16_bits_to_f32(a.conv1[(size_t)c * 9 + k]));
+        v = fmaxf(v, fabsf(a.bias1[c]) + sum * bound);
     }
-    emit(bound, scales);
-    if (!a.norms2) return;
+    bound = block_max_256(v, red);
     v = 0.0f;
     for (uint32_t c = threadIdx.x; c < a.channels; c += 256) v = fmaxf(v, fabsf(a.bias2[c]) + a.norms2[c] * bound);
-    emit(block_max_256(v, red), scales + 2);
+    const float next = block_max_256(v, red);
+    if (threadIdx.x == 0) {
+        const float2 first = scale_of(bound), second = scale_of(next);
+        reinterpret_cast<float4 *>(a.scales)[blockIdx.x] = make_float4(first.x, first.y, second.x, second.y);
+    }
 }
 
 // f32 [image][channel][h][w] to the halves layout, border included: a thread
-// per word pair (both terms), channels in groups of eight.
+// per word pair (both terms), channels in groups of eight. Each workgroup takes
+// its image's scale from the (at most 256) partial maxima; an image's first
+// one stores it.
 __global__ __launch_bounds__(256) void to_halves_kernel(const float *in, uint32_t channels, uint32_t h, uint32_t w,
-                                                        const float *scales, uint8_t *out) {  // (scales: an image's two)
+                                                        const float *partial, uint32_t partials, float *scales,
+                                                        uint8_t *out) {
+    __shared__ float red[4];
     const HalvesPlane p = halves_plane(h, w);
+    const float2 scale = scale_of(block_max_256(
+        threadIdx.x < partials ? partial[(size_t)blockIdx.z * partials + threadIdx.x] : 0.0f, red));
+    if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) reinterpret_cast<float2 *>(scales)[blockIdx.z] = scale;
     const uint32_t i = blockIdx.x * 256 + threadIdx.x;
     if (i >= p.words) return;
     const uint32_t c0 = blockIdx.y * 8, b = blockIdx.z;
     const uint32_t row = i / (2 * p.slots), rest = i % (2 * p.slots);
     const uint32_t col = 2 * (rest % p.slots) + rest / p.slots;
     const bool inside = row >= 1 && row <= h && col >= 1 && col <= w;
-    const float up = scales[2 * (size_t)b];
+    const float up = scale.x;
     const float *src = in + (((size_t)b * channels + c0) * h + (inside ? row - 1 : 0)) * w + (inside ? col - 1 : 0);
     ch8 hi, lo;
 #pragma unroll
@@ -781,16 +795,23 @@ uint32_t mfma_patch_rows(uint32_t ow, uint32_t positions = kMfPos) { return 2 * 
 
 uint32_t mfma_oc_pad(uint32_t out_ch) { return (out_ch + 63) / 64 * 64; }
 
-// Workgroups that look for an image's largest magnitude: four rows a wavefront
-// and more.
-uint32_t maxima_blocks(uint32_t rows) { return std::min(16u, (rows + 15) / 16); }
+// Workgroups that look for an image's largest magnitude: four rows a wavefront,
+// more of them where the images alone fill the device; at most 256 to an image.
+uint32_t maxima_blocks(uint32_t images, uint32_t rows) {
+    return std::min({(rows + 15) / 16, std::max(1u, 2048 / images), 256u});
+}
+// An image that lies in one piece is read in rows of this many values.
+constexpr uint32_t kMaximaRow = 256;
+uint32_t maxima_rows(uint32_t channels, uint32_t h, uint32_t w) {
+    return (uint32_t)(((uint64_t)channels * h * w + kMaximaRow - 1) / kMaximaRow);
+}
 
 // Workspace pieces of a prepared convolution: operand-order weights, channel
 // sums, partial maxima and scales, 256-byte aligned.
 size_t piece(size_t bytes) { return (bytes + 255) & ~(size_t)255; }
 size_t wprep_bytes(uint32_t out_ch, uint32_t in_ch) { return piece((size_t)mfma_oc_pad(out_ch) * in_ch * 9 * 2); }
 size_t norms_bytes(uint32_t out_ch) { return piece((size_t)mfma_oc_pad(out_ch) * sizeof(float)); }
-size_t maxima_bytes(uint32_t images, uint32_t rows) { return piece((size_t)images * maxima_blocks(rows) * sizeof(float)); }
+size_t maxima_bytes(uint32_t images, uint32_t rows) { return piece((size_t)images * maxima_blocks(images, rows) * sizeof(float)); }
 size_t scale_bytes(uint32_t images) { return piece((size_t)images * 4 * sizeof(float)); }
 
 size_t halves_image_bytes(uint32_t channels, uint32_t h, uint32_t w) {
@@ -886,7 +907,7 @@ uint32_t conv_mfma_group(uint32_t batch, uint32_t in_ch, uint32_t h, uint32_t w)
 }
 
 size_t conv_mfma_bytes(int cus, uint32_t batch, uint32_t out_ch, uint32_t in_ch, uint32_t h, uint32_t w) {
-    return wprep_bytes(out_ch, in_ch) + norms_bytes(out_ch) + maxima_bytes(batch, in_ch) + scale_bytes(batch) +
+    return wprep_bytes(out_ch, in_ch) + norms_bytes(out_ch) + maxima_bytes(batch, maxima_rows(in_ch, h, w)) + scale_bytes(batch) +
            conv_part_bytes(cus) +
            conv_mfma_group(batch, in_ch, h, w) * halves_image_bytes(in_ch, h, w);
 }
@@ -899,30 +920,26 @@ hipError_t launch_conv3x3s2_gelu_mfma(hipStream_t s, int cus, float *out, const 
     uint8_t *wprep = at;
     float *norms = reinterpret_cast<float *>(at += wprep_bytes(out_ch, in_ch));
     float *partial = reinterpret_cast<float *>(at += norms_bytes(out_ch));
-    float *scales = reinterpret_cast<float *>(at += maxima_bytes(batch, in_ch));
+    float *scales = reinterpret_cast<float *>(at += maxima_bytes(batch, maxima_rows(in_ch, h, w)));
     float *part = reinterpret_cast<float *>(at += scale_bytes(batch));
     uint8_t *halves = at + conv_part_bytes(cus);
     ConvPrepArgs p{};
     p.job[0] = {weights, wprep, norms, out_ch, mfma_oc_pad(out_ch), in_ch};
     p.x = in;
-    p.rows = in_ch;
-    p.row_values = p.row_stride = (uint64_t)h * w;
-    p.image_stride = in_ch * p.row_stride;
-    p.row_limit = batch * p.image_stride;
+    p.rows = maxima_rows(in_ch, h, w);
+    p.row_values = kMaximaRow;
+    p.row_stride = p.row_used = kMaximaRow;
+    p.image_stride = p.limit = (uint64_t)in_ch * h * w;
     p.partial = partial;
-    p.partials = maxima_blocks(in_ch);
+    p.partials = maxima_blocks(batch, p.rows);
     conv_prep_kernel<<<p.job[0].oc_pad + batch * p.partials, 256, 0, s>>>(p);
-    ConvScaleArgs c{};
-    c.partial = partial;
-    c.partials = p.partials;
-    c.scales = scales;
-    conv_scale_kernel<<<batch, 256, 0, s>>>(c);
     ConvMfmaArgs a = mfma_args(halves, wprep, bias, scales, 2, out_ch, in_ch, h, w);
     const uint32_t group = conv_mfma_group(batch, in_ch, h, w);
     for (uint32_t b = 0; b < batch; b += group) {
         const uint32_t n = std::min(group, batch - b);
         to_halves_kernel<<<dim3((halves_plane(h, w).words + 255) / 256, in_ch / 8, n), 256, 0, s>>>(
-            in + (size_t)b * in_ch * h * w, in_ch, h, w, scales + 2 * (size_t)b, halves);
+            in + (size_t)b * in_ch * h * w, in_ch, h, w, partial + (size_t)b * p.partials, p.partials,
+            scales + 2 * (size_t)b, halves);
         a.scales = scales + 2 * (size_t)b;
         a.out = out + (size_t)b * out_ch * a.positions;
         const hipError_t e = launch_mfma<false>(s, cus, a, n, part);
@@ -980,10 +997,11 @@ hipError_t launch_conv_tower_prep(hipStream_t s, int cus, const ConvTower &c, co
     p.job[1] = {c.weights[2], base + at.wprep3, reinterpret_cast<float *>(base + at.norms3), c.channels, pad, c.channels};
     p.x = mel;
     p.rows = c.bins;
-    p.row_values = p.image_stride = c.chunk_frames;
-    p.row_stride = p.row_limit = frames;
+    p.row_values = c.chunk_frames;
+    p.image_stride = p.image_used = c.chunk_frames;
+    p.row_stride = p.limit = frames;
     p.partial = reinterpret_cast<float *>(base + at.partial);
-    p.partials = maxima_blocks(c.bins);
+    p.partials = maxima_blocks(c.chunks, c.bins);
     conv_prep_kernel<<<2 * pad + c.chunks * p.partials, 256, 0, s>>>(p);
     ConvScaleArgs q{};
     q.partial = p.partial;
