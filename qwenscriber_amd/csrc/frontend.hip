@@ -811,7 +811,11 @@ uint32_t maxima_rows(uint32_t channels, uint32_t h, uint32_t w) {
 size_t piece(size_t bytes) { return (bytes + 255) & ~(size_t)255; }
 size_t wprep_bytes(uint32_t out_ch, uint32_t in_ch) { return piece((size_t)mfma_oc_pad(out_ch) * in_ch * 9 * 2); }
 size_t norms_bytes(uint32_t out_ch) { return piece((size_t)mfma_oc_pad(out_ch) * sizeof(float)); }
-size_t maxima_bytes(uint32_t images, uint32_t rows) { return piece((size_t)images * maxima_blocks(images, rows) * sizeof(float)); }
+// (At least images * maxima_blocks, and no less for more images: a caller sizes for
+// its largest run.)
+size_t maxima_bytes(uint32_t images, uint32_t rows) {
+    return piece(std::min<size_t>((size_t)images * std::min((rows + 15) / 16, 256u), std::max(images, 2048u)) * sizeof(float));
+}
 size_t scale_bytes(uint32_t images) { return piece((size_t)images * 4 * sizeof(float)); }
 
 size_t halves_image_bytes(uint32_t channels, uint32_t h, uint32_t w) {
