@@ -209,7 +209,8 @@ int32_t qwh_linear(qwh_ctx *ctx, uint64_t matrix, const float *x_dev, uint32_t c
  * same activations (decoder.zig:174-176 applies q, k and v to one `normed`
  * row): qwh_activation_prepare encodes x once into `prepared_dev` (at least
  * qwh_activation_bytes(cols, tokens) bytes), qwh_linear_prepared multiplies a
- * q4 matrix by it. The results equal qwh_linear's. */
+ * q4 matrix by it. The results equal qwh_linear's for one token, and for more
+ * within rounding (it may take another form). */
 int32_t qwh_activation_bytes(uint32_t cols, uint32_t tokens, uint64_t *out_bytes);
 int32_t qwh_activation_prepare(qwh_ctx *ctx, const float *x_dev, uint32_t cols, uint32_t tokens,
                                void *prepared_dev);

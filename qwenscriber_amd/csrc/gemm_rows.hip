@@ -5,8 +5,8 @@
 // Each token's row is split once into two f16 terms of x * 2^s (s from the
 // row's largest finite magnitude, so |x * 2^s| < 2^14): hi rounded to f16, lo
 // the exact remainder rounded to f16. A value is kept to 2^-22 of itself or
-// 2^-39 of what s was taken from, whichever is more. A row with a 64-value
-// group 2^-15 or more below its largest takes s from each group instead (an
+// 2^-39 of what s was taken from, whichever is more. A row with a 64-value group
+// more than 2^15 below its largest takes s from each group instead (an
 // "uneven" row), so the split is at least as close as 23-bit integers per group
 // (the small batch's digit planes) whatever the row holds: one s for a row with
 // a value 1e8 times the others left them 1e-4 of themselves. The codes are
@@ -14,7 +14,7 @@
 // matrix core adds both terms' products of one group into one f32 partial,
 // which takes the group's f16 scale in one FMA, in a workgroup with an uneven
 // row times the token's 2^-s (2048 x 6144 q8 and 12288 x 2048 q4 at 402 tokens:
-// 44.9 and 58.1 us, 47.1 and 68.0 with all rows uneven).
+// 43.1 and 57.2 us, 46.4 and 67.0 with all rows uneven).
 //
 // Operands. One v_mfma_f32_32x32x16_f16 multiplies 32 tokens by 32 weight
 // rows over 16 columns: lane l feeds token (or row) l % 32 and 8 columns, so
@@ -31,12 +31,14 @@
 // With the tokens as the result's rows, a lane's 16 results of a tile belong
 // to one weight row: one scale per lane and group.
 //
-// Bound by the matrix cores' and the vector unit's shared issue: two products
-// per weight, and per group the decode and 16 scale FMAs a tile. 12288 x 2048
-// q4 at 2048 tokens runs at 440-475 TFLOP/s (twice that in f16 products, of
-// the 1.2 PFLOP/s an 8192^3 f16 matmul reaches on the same card); at 402 tokens
-// at 375, the last wave of workgroups partly empty. Tiles of 64 rows or 128
-// tokens a wavefront, or eight wavefronts, measured within 10 %.
+// Where a SIMD has two and more wavefronts, near the shared issue of matrix cores
+// and vector unit (two products per weight, and per group the decode and 16
+// scale FMAs a tile): 12288 x 2048 q4 at 402 tokens keeps them busy 32 and 40 %
+// of the cycles, 370 TFLOP/s, and at 2048 tokens reaches 440-475 (twice that in
+// f16 products, of the 1.2 PFLOP/s an 8192^3 f16 matmul reaches on the same
+// card). With one or two a SIMD it waits for its own loads and barriers: 4096 x
+// 2048 18 and 19 %, 2048 x 2048 14 and 17 %. No LDS bank conflicts. Tiles of 64
+// rows or 128 tokens a wavefront, or eight wavefronts, measured within 10 %.
 #include <algorithm>
 #include <cmath>
 #include <type_traits>
@@ -303,7 +305,7 @@ __device__ __forceinline__ void rows_block(const RowsArgs &a, uint32_t row_block
     };
     if (uneven) {
         // A group at a time, the next one's codes and multipliers loaded
-        // meanwhile (5 to 17 % slower than the loop below).
+        // meanwhile (8 to 17 % slower than the loop below).
         const float *mp = a.uneven + (size_t)(my_token / kTile) * a.groups * kTile + my_token % kTile;
         uint16_t next_s = sp[g0];
         float next_m = mp[(size_t)g0 * kTile];
