@@ -14,7 +14,7 @@
 // matrix core adds both terms' products of one group into one f32 partial,
 // which takes the group's f16 scale in one FMA, in a workgroup with an uneven
 // row times the token's 2^-s (2048 x 6144 q8 and 12288 x 2048 q4 at 402 tokens:
-// 43.1 and 57.2 us, 46.4 and 67.0 with all rows uneven).
+// 43.4 and 58.1 us, 47.0 and 68.2 with all rows uneven).
 //
 // Operands. One v_mfma_f32_32x32x16_f16 multiplies 32 tokens by 32 weight
 // rows over 16 columns: lane l feeds token (or row) l % 32 and 8 columns, so
@@ -170,7 +170,7 @@ __device__ __forceinline__ void rows_block(const RowsArgs &a, uint32_t row_block
     constexpr int D = 3;
     __shared__ u4 al[D][PIECES];
     __shared__ float inv[TT * kTile];
-    __shared__ float4 mult[W][64 / 4];  // a group's 2^-s by token, a copy for each wavefront
+    __shared__ __attribute__((aligned(16))) float mult[W][64];  // a group's 2^-s by token, a copy for each wavefront
     const int tid = threadIdx.x;
     const int lane = tid & 63, wave = tid >> 6;
     const int col = lane & 31, half = lane >> 5;
@@ -317,7 +317,7 @@ __device__ __forceinline__ void rows_block(const RowsArgs &a, uint32_t row_block
 #pragma unroll
             for (int k = 0; k < CW; ++k) w[k] = rw[0][k];
             const float sv = dev::f16_bits_to_f32(next_s);
-            reinterpret_cast<float *>(mult[wave])[lane] = my_scale == 0.0f ? next_m : my_scale;
+            mult[wave][lane] = my_scale == 0.0f ? next_m : my_scale;
             const uint32_t gn = min(g + 1, g1 - 1);
             load_codes<C>(wp + (size_t)gn * code_bytes(C), half, rw[0]);
             next_s = sp[gn];
@@ -329,11 +329,9 @@ __device__ __forceinline__ void rows_block(const RowsArgs &a, uint32_t row_block
             for (int t = 0; t < TT; ++t)
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
-                    const float4 q = mult[wave][t * 8 + 2 * j + half];
-                    acc[t][4 * j] = fmaf(p[t][4 * j], sv * q.x, acc[t][4 * j]);
-                    acc[t][4 * j + 1] = fmaf(p[t][4 * j + 1], sv * q.y, acc[t][4 * j + 1]);
-                    acc[t][4 * j + 2] = fmaf(p[t][4 * j + 2], sv * q.z, acc[t][4 * j + 2]);
-                    acc[t][4 * j + 3] = fmaf(p[t][4 * j + 3], sv * q.w, acc[t][4 * j + 3]);
+                    const float *q = &mult[wave][t * kTile + 8 * j + 4 * half];
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) acc[t][4 * j + k] = fmaf(p[t][4 * j + k], sv * q[k], acc[t][4 * j + k]);
                 }
             buf = buf == D - 1 ? 0 : buf + 1;
         }

@@ -93,3 +93,19 @@ def test_conv_outlier_within_an_image(ctx, outlier):
     away = np.ones((8, 8), bool)
     away[2:4, 2:4] = False
     assert_close(got[:, away], want[:, away], rtol=2e-5, atol_rms=2e-5)
+
+
+def test_conv_runs_of_images(ctx):
+    # More images than their terms' scratch holds at once (38 of this shape):
+    # the second run's images take their own scales.
+    cin, cout, h, w, batch = 480, 32, 64, 50, 40
+    two = normal(2 * cin * h * w, 104, 0).reshape(2, cin, h, w)
+    two[1] *= np.float32(1e9)
+    x = np.concatenate([two] * (batch // 2))
+    wb = f16_fast(normal(cout * cin * 9, 105, 0, 1.0 / np.sqrt(9 * cin)))
+    b = normal(cout, 106, 0, 0.1)
+    got = run_conv(ctx, x.reshape(-1), wb, b, batch, cout, cin, h, w)
+    for i in range(2):
+        want = o.conv3x3s2_gelu(two[i].reshape(-1), wb, b, cout, cin, h, w)
+        for k in (i, 36 + i, 38 + i):
+            assert_close(got[k], want, rtol=1e-5, atol_rms=1e-5, what=f"image {k}")
